@@ -3640,15 +3640,21 @@ int edlut_network_get_stdp(edlut_network *n, int source, float *pre, float *post
 }  // extern "C"
 
 struct edlut_fit {
-    int model = 0, n = 0, steps = 0, n_syn = 0, ckpt = 100, device = 0;
+    int model = 0, n = 0, steps = 0, n_syn = 0, device = 0;
     FitArgs base{};
+    int group = 0;                 // segments the backward pass takes per launch
     float *refr = nullptr;
     float *ck_state = nullptr;
     int32_t *ck_int = nullptr;
-    float *scratch = nullptr;
-    int32_t *scratch_int = nullptr;
+    double *maps = nullptr, *part = nullptr, *carry = nullptr;
+    float *lg = nullptr;
     bool forward_done = false;
 };
+
+// Working storage of a backward launch: its segments' maps, partial
+// gradients and conductance adjoints.  Past this the pass takes several
+// launches, last segments first.
+static constexpr size_t kFitScratch = (size_t)256 << 20;
 
 extern "C" {
 
@@ -3681,15 +3687,14 @@ int edlut_fit_create(int model, const float *params, int n_params, float dt_s, i
     f->n = n_neurons;
     f->steps = steps;
     f->n_syn = n_syn;
-    f->ckpt = checkpoint < steps ? checkpoint : steps;
     f->device = device;
     FitArgs &a = f->base;
     std::memset(&a, 0, sizeof(a));
-    a.model = model == EDLUT_LIF ? 0 : 1;
     a.n = n_neurons;
     a.steps = steps;
     a.n_syn = n_syn;
-    a.ckpt = f->ckpt;
+    a.seg = std::min(std::min(checkpoint, steps), kFitSeg);
+    a.segs = (steps + a.seg - 1) / a.seg;
     a.dt = dt_s * 1000.0f;
     a.h = model == EDLUT_ADEX ? a.dt * 0.5f : a.dt;
     a.s6 = a.dt * 0.166666666667f;
@@ -3716,12 +3721,15 @@ int edlut_fit_create(int model, const float *params, int n_params, float dt_s, i
         a.v_cap = params[3] + 6 * params[2];
     }
     a.refr_len = (int)refr.size();
-    const int segs = (steps + f->ckpt - 1) / f->ckpt;
+    const size_t n = (size_t)n_neurons, segs = (size_t)a.segs;
+    const size_t per_seg = n * (sizeof(double) * (kFitMap + 4) + sizeof(float) * 2 * a.seg);
+    f->group = (int)std::max<size_t>(1, std::min(segs, kFitScratch / per_seg));
+    const size_t group = (size_t)f->group;
     int rc;
-    if ((rc = dalloc(&f->refr, refr.size() + 1)) || (rc = dalloc(&f->ck_state, (size_t)(segs + 1) * 4 * n_neurons)) ||
-        (rc = dalloc(&f->ck_int, (size_t)(segs + 1) * 2 * n_neurons)) ||
-        (rc = dalloc(&f->scratch, (size_t)f->ckpt * kFitStore * n_neurons)) ||
-        (rc = dalloc(&f->scratch_int, (size_t)f->ckpt * n_neurons))) {
+    if ((rc = dalloc(&f->refr, refr.size() + 1)) || (rc = dalloc(&f->ck_state, segs * 4 * n)) ||
+        (rc = dalloc(&f->ck_int, (segs + 1) * 2 * n)) || (rc = dalloc(&f->maps, group * kFitMap * n)) ||
+        (rc = dalloc(&f->part, group * 4 * n)) || (rc = dalloc(&f->lg, group * a.seg * 2 * n)) ||
+        (rc = dalloc(&f->carry, 8 * n))) {
         edlut_fit_destroy(f);
         return rc;
     }
@@ -3733,8 +3741,10 @@ int edlut_fit_create(int model, const float *params, int n_params, float dt_s, i
     a.refr = f->refr;
     a.ck_state = f->ck_state;
     a.ck_int = f->ck_int;
-    a.scratch = f->scratch;
-    a.scratch_int = f->scratch_int;
+    a.maps = f->maps;
+    a.part = f->part;
+    a.lg = f->lg;
+    a.carry = f->carry;
     *out = f;
     return 0;
 }
@@ -3743,7 +3753,7 @@ int edlut_fit_destroy(edlut_fit *f) {
     if (!f) return 0;
     (void)hipSetDevice(f->device);
     (void)hipDeviceSynchronize();
-    void *dev[] = {f->refr, f->ck_state, f->ck_int, f->scratch, f->scratch_int};
+    void *dev[] = {f->refr, f->ck_state, f->ck_int, f->maps, f->part, f->lg, f->carry};
     for (void *q : dev)
         if (q) (void)hipFree(q);
     delete f;
@@ -3784,7 +3794,10 @@ int edlut_fit_forward(edlut_fit *f, const edlut_fit_tensors *t, void *stream) {
     if (!t->v_trace) return fail(EDLUT_E_ARG, "v_trace is null");
     HIP_TRY(hipSetDevice(f->device));
     const int blocks = (f->n + kFitBlock - 1) / kFitBlock;
-    hipLaunchKernelGGL(k_fit_forward, dim3(blocks), dim3(kFitBlock), 0, (hipStream_t)stream, a);
+    const bool extra = t->spikes || t->traj || a.refr_len > kFitRefr;
+    auto fn = f->model == EDLUT_LIF ? (extra ? k_fit_forward<0, true> : k_fit_forward<0, false>)
+                                    : (extra ? k_fit_forward<1, true> : k_fit_forward<1, false>);
+    hipLaunchKernelGGL(fn, dim3(blocks), dim3(2 * kFitBlock), 0, (hipStream_t)stream, a);
     HIP_TRY(hipGetLastError());
     f->forward_done = true;
     return 0;
@@ -3797,8 +3810,20 @@ int edlut_fit_backward(edlut_fit *f, const edlut_fit_tensors *t, void *stream) {
     if (!t->grad_v || !t->grad_par || !t->grad_w) return fail(EDLUT_E_ARG, "gradient tensors are null");
     if (!f->forward_done) return fail(EDLUT_E_STATE, "the backward pass needs the forward pass's checkpoints");
     HIP_TRY(hipSetDevice(f->device));
-    const int blocks = (f->n + kFitBlock - 1) / kFitBlock;
-    hipLaunchKernelGGL(k_fit_backward, dim3(blocks), dim3(kFitBlock), 0, (hipStream_t)stream, a);
+    const hipStream_t st = (hipStream_t)stream;
+    const bool lif = f->model == EDLUT_LIF;
+    const unsigned neurons = (unsigned)((f->n + kFitBlock - 1) / kFitBlock);
+    // the adjoint state after the last step is zero
+    hipLaunchKernelGGL(k_fill_i32, dim3(std::min(neurons, 1024u)), dim3(kBlock), 0, st, (int32_t *)f->carry,
+                       (int64_t)(2 * 4) * f->n, 0);
+    for (a.c_hi = a.segs; a.c_hi > 0; a.c_hi = a.c_lo) {
+        a.c_lo = std::max(a.c_hi - f->group, 0);
+        const unsigned blocks = (unsigned)(((int64_t)(a.c_hi - a.c_lo) * f->n + kFitBlock - 1) / kFitBlock);
+        hipLaunchKernelGGL(lif ? k_fit_maps<0> : k_fit_maps<1>, dim3(blocks), dim3(kFitBlock), 0, st, a);
+        hipLaunchKernelGGL(k_fit_scan, dim3(neurons), dim3(kFitBlock), 0, st, a);
+        hipLaunchKernelGGL(lif ? k_fit_sweep<0> : k_fit_sweep<1>, dim3(blocks), dim3(kFitBlock), 0, st, a);
+        hipLaunchKernelGGL(k_fit_grads, dim3((unsigned)f->n), dim3(kFitGradBlock), 0, st, a);
+    }
     HIP_TRY(hipGetLastError());
     return 0;
 }

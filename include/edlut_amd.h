@@ -429,7 +429,7 @@ int edlut_network_autotune(edlut_network *net, int trial_steps, int *items, int 
  * dt_s.  params holds the model's parameter vector (order of
  * edlut_population_create); g_leak, e_leak, tau_exc and tau_inh are taken
  * per neuron from the tensors instead.  The forward pass writes the V trace
- * and keeps the state every `checkpoint` steps; the backward pass takes
+ * and keeps the state every `checkpoint` steps (32 at most); the backward pass takes
  * dL/dV for every step and writes dL/d(g_leak, e_leak, tau_exc, tau_inh)
  * per neuron and dL/dweight per synapse.  It is the reverse-mode derivative
  * of the discrete forward map, with the forward run's spike pattern held
