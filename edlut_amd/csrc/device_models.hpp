@@ -944,57 +944,6 @@ __device__ __forceinline__ void integrate_bdf(const ModelParams &mp, const RhsCt
 }
 
 // ---------------------------------------------------------------------------
-// Granule BDF step (the same algorithm as integrate_bdf, BDFn.h:288-423 and
-// 682-786), arranged for a 15-variable system held in registers:
-//   * the Jacobian column of a gate perturbs one variable: only the rows
-//     whose equations read it are evaluated (the others difference to +0
-//     exactly, as in the reference), and the table row and the Nernst
-//     potential are reused unless V or Ca is the perturbed variable;
-//   * the inverse is formed in place: at pivot s the dead column s of the
-//     eliminated matrix becomes column s of the inverse, and the inverse's
-//     still-unit columns are not stored.  Every stored value takes exactly
-//     the reference's operations (li[i][s] = 0 + li[s][s]*coef included);
-//   * a zero pivot (the reference then swaps rows) or a non-finite value
-//     sends that Newton iteration through the reference arrangement
-//     (granule_newton_reference) on a global working-storage slot, so that
-//     the kernel keeps no large private frame.
-// ---------------------------------------------------------------------------
-template <int N>
-__device__ __forceinline__ bool invert_in_place(float *A) {
-    bool ok = true;
-#pragma unroll
-    for (int s = 0; s < N; s++) {
-        const float element = A[s * N + s];
-        ok = ok && element != 0.0f;
-        const float inv = 1.0f / element;
-#pragma unroll
-        for (int j = 0; j < N; j++)
-            if (j != s) A[s * N + j] *= inv;
-        A[s * N + s] = inv;
-#pragma unroll
-        for (int i = 0; i < N; i++) {
-            if (i == s) continue;
-            const float coef = -A[i * N + s];
-#pragma unroll
-            for (int j = 0; j < N; j++)
-                if (j != s) A[i * N + j] += A[s * N + j] * coef;
-            A[i * N + s] = 0.0f + A[s * N + s] * coef;
-        }
-    }
-    bool fin = true;
-#pragma unroll
-    for (int q = 0; q < N * N; q++) fin = fin && __builtin_isfinite(A[q]);
-    return ok && fin;
-}
-
-template <int N>
-__device__ __forceinline__ bool any_nan(const float *x) {
-    bool r = false;
-#pragma unroll
-    for (int q = 0; q < N; q++) r = r || x[q] != x[q];
-    return r;
-}
-
 // Floats of one working-storage slot: la, li (15 x 15 each), X (19), Fp, Fn,
 // Cc, P1 (15 each).
 constexpr int kGrWsFloats = 2 * 225 + 19 + 4 * 15;
@@ -1058,179 +1007,6 @@ __device__ __forceinline__ void granule_newton_reference(const ModelParams &mp, 
         for (int t = 0; t < ND; t++) aux += li[z * ND + t] * (X[t] - Cc[t]);
         P1[z] = aux + X[z];
     }
-}
-
-// The granule BDF step in three parts, so that the update kernel can hand a
-// lane its next neuron as soon as that lane's corrector has converged:
-// granule_bdf_predict (the order-st predictor), granule_bdf_newton (one
-// corrector iteration, repeated while epsi > 1e-6 and k < 10) and
-// granule_bdf_commit (history shift and new state).  Run in that order they
-// are the step of integrate_bdf above, BDFn.h:288-423.  The corrector reads
-// the first previous-state row from ph0 (a lane's copy in LDS, stride kBlock,
-// taken when the lane took the neuron), the older rows from memory.
-template <unsigned MASK>
-__device__ __forceinline__ void granule_bdf_predict(const ModelParams &mp, const RhsCtx &c, float dt,
-                                                    const BdfState &b, int64_t ld, uint32_t i, int st,
-                                                    const float *S, float *P) {
-    using G = GranuleModel;
-    constexpr int ND = G::ND, NV = G::NV;
-    const float *Dh = (const float *)b.d;
-    if (st == 0) {
-        float F[ND];
-        G::rhs<MASK>(mp, c, (float *)S, F);
-#pragma unroll
-        for (int j = 0; j < ND; j++) P[j] = S[j] + dt * F[j];
-    } else {
-#pragma unroll
-        for (int j = 0; j < ND; j++) {
-            P[j] = S[j];
-            for (int q = 0; q < st; q++) P[j] += Dh[((int64_t)q * ND + j) * ld + i];
-        }
-    }
-#pragma unroll
-    for (int j = ND; j < NV; j++) P[j] = S[j];
-    G::decay<MASK>(mp, P);
-}
-
-template <unsigned MASK>
-__device__ __forceinline__ void granule_bdf_newton(const ModelParams &mp, const RhsCtx &c, float dt,
-                                                   const BdfState &b, int par, int64_t ld, uint32_t i, int st,
-                                                   const float *S, float *P, float &epsi, int &k,
-                                                   const float *ph0) {
-    using G = GranuleModel;
-    constexpr int ND = G::ND, NV = G::NV;
-    const float *Ph = (const float *)b.prev;
-    float F[ND], P1[ND], Cc[ND], A[ND * ND];
-    const float *Cs = b.C + st * 7;
-    const float c0 = Cs[0], c0dt = c0 * dt;
-    const float eps = dt * 0.1f;
-    const float inv_eps = 1.0f / eps;
-    {
-        G::Terms t;
-        G::prep(mp, c, P, t);
-        G::rhs_terms(mp, c, P, t, F);
-        bool fin = true;
-#pragma unroll
-        for (int j = 0; j < ND; j++) {
-            Cc[j] = c0 * dt * F[j] + Cs[1] * S[j];
-            if (st > 1) Cc[j] += Cs[2] * ph0[j * kBlock];
-            for (int q = 2; q < st; q++) Cc[j] += Cs[q + 1] * Ph[((int64_t)(q - 1) * ND + j) * ld + i];
-            fin = fin && __builtin_isfinite(F[j]);
-        }
-        // J = c0*dt*jac - I, jac[z][j] = (F[z] - Fn_j[z]) / eps (one-sided, at P)
-#pragma unroll
-        for (int q = 0; q < ND * ND; q++) A[q] = 0.0f;
-        {   // V: every equation reads it (table row at the perturbed V)
-            float X[NV], Fn[ND];
-            G::Terms tv;
-#pragma unroll
-            for (int q = 0; q < NV; q++) X[q] = P[q];
-            X[0] -= eps;
-            G::load_row(c, X[0], tv.v);
-            tv.vca = t.vca;
-            G::rhs_terms(mp, c, X, tv, Fn);
-#pragma unroll
-            for (int z = 0; z < ND; z++) A[z * ND] = c0dt * ((F[z] - Fn[z]) * inv_eps);
-        }
-#pragma unroll
-        for (int j = 1; j < 14; j++) {   // gates: the membrane equation and their own (+ calcium for xCa, yCa)
-            float X[NV];
-#pragma unroll
-            for (int q = 0; q < NV; q++) X[q] = P[q];
-            X[j] -= eps;
-            A[j] = c0dt * ((F[0] - G::dv(mp, c, X, t.vca)) * inv_eps);
-            const float fj = j == 10 ? G::dxkca(mp.gran, X, t.v) : G::dgate(j, X, t.v);
-            A[j * ND + j] = c0dt * ((F[j] - fj) * inv_eps);
-            if (j == 11 || j == 12) A[14 * ND + j] = c0dt * ((F[14] - G::dca(X, t.vca)) * inv_eps);
-        }
-        {   // Ca: the membrane equation (Nernst potential), the Ca-dependent K gate, calcium
-            float X[NV];
-#pragma unroll
-            for (int q = 0; q < NV; q++) X[q] = P[q];
-            X[14] -= eps;
-            const float vca = G::nernst_ca(mp.gran, X[14]);
-            A[14] = c0dt * ((F[0] - G::dv(mp, c, X, vca)) * inv_eps);
-            A[10 * ND + 14] = c0dt * ((F[10] - G::dxkca(mp.gran, X, t.v)) * inv_eps);
-            A[14 * ND + 14] = c0dt * ((F[14] - G::dca(X, vca)) * inv_eps);
-        }
-#pragma unroll
-        for (int z = 0; z < ND; z++) A[z * ND + z] -= 1;
-        if (fin && invert_in_place<ND>(A)) {
-#pragma unroll
-            for (int z = 0; z < ND; z++) {
-                float aux = 0.0f;
-#pragma unroll
-                for (int q = 0; q < ND; q++) aux += A[z * ND + q] * (P[q] - Cc[q]);
-                P1[z] = aux + P[z];
-            }
-        } else if (any_nan<ND>(P)) {
-            // An iterate with a NaN component corrects to all NaN whatever
-            // the Jacobian: every P1[z] = sum_t iJ[z][t] * (P[t] - Cc[t]) +
-            // P[z] takes the NaN term (and the max-norm change below is then
-            // 0: no comparison with a NaN holds).  This is the standing case
-            // of a neuron whose step once went NaN: the NaN reset restores
-            // the state but not the BDF history (TimeDrivenNeuronModel.cpp:
-            // 75-88), so every later predictor is NaN.  Only the NaN payload
-            // can differ from the full correction's.
-#pragma unroll
-            for (int q = 0; q < ND; q++) P1[q] = __builtin_nanf("");
-        } else {
-            const uint32_t slot = atomicAdd(&b.ws_count[par], 1u);
-            if (slot < (uint32_t)b.ws_cap) {
-                float *w = b.ws + (size_t)slot * kGrWsFloats;
-                float *X = w + 450, *Cw = X + NV + 2 * ND, *P1w = Cw + ND;
-#pragma unroll
-                for (int q = 0; q < NV; q++) X[q] = P[q];
-#pragma unroll
-                for (int q = 0; q < ND; q++) Cw[q] = Cc[q];
-                granule_newton_reference(mp, c, dt, c0, w);
-#pragma unroll
-                for (int q = 0; q < ND; q++) P1[q] = P1w[q];
-            } else {
-                atomicOr(b.err, 16u);   // reported to the host; the step is not the reference's
-#pragma unroll
-                for (int q = 0; q < ND; q++) P1[q] = P[q];
-            }
-        }
-        float aux2 = 0.0f;
-#pragma unroll
-        for (int z = 0; z < ND; z++) {
-            const float aux = fabsf(P1[z] - P[z]);
-            if (aux > aux2) aux2 = aux;
-        }
-#pragma unroll
-        for (int z = 0; z < ND; z++) P[z] = P1[z];
-        epsi = aux2;
-        k++;
-    }
-}
-
-template <unsigned MASK>
-__device__ __forceinline__ void granule_bdf_commit(const ModelParams &mp, const BdfState &b, int64_t ld,
-                                                   uint32_t i, int &st, float *S, const float *P) {
-    using G = GranuleModel;
-    constexpr int ND = G::ND;
-    float *Dh = (float *)b.d;
-    float *Ph = (float *)b.prev;
-    if (st < b.order) st++;
-#pragma unroll
-    for (int j = 0; j < ND; j++) {
-        for (int q = st - 1; q > 0; q--) Dh[((int64_t)q * ND + j) * ld + i] = -Dh[((int64_t)(q - 1) * ND + j) * ld + i];
-        Dh[(int64_t)j * ld + i] = P[j] - S[j];
-        for (int q = 1; q < st; q++)
-            Dh[((int64_t)q * ND + j) * ld + i] += Dh[((int64_t)(q - 1) * ND + j) * ld + i];
-    }
-    if (st > 1) {
-        for (int q = st - 2; q > 0; q--)
-#pragma unroll
-            for (int j = 0; j < ND; j++)
-                Ph[((int64_t)q * ND + j) * ld + i] = Ph[((int64_t)(q - 1) * ND + j) * ld + i];
-#pragma unroll
-        for (int j = 0; j < ND; j++) Ph[(int64_t)j * ld + i] = S[j];
-    }
-#pragma unroll
-    for (int j = 0; j < ND; j++) S[j] = P[j];
-    G::decay<MASK>(mp, S);
 }
 
 }  // namespace edl

@@ -18,6 +18,7 @@
 #include "../../include/edlut_amd.h"
 #include "adjoint.hpp"
 #include "generate.hpp"
+#include "granule_bdf.hpp"
 #include "kernels.hpp"
 
 using namespace edl;
@@ -337,12 +338,27 @@ struct edlut_population {
     int items = kItems;              // neurons per thread of the update launch
 
     int update_tiles() const { return (int)(stride / ((int64_t)kBlock * items)); }
+    bool granule_bdf() const { return model == EDLUT_GRANULE && integ == EDLUT_BDF; }
+    // waves that give every neuron its kGrLanes lanes at once
+    int granule_waves() const { return (int)(((int64_t)n * kGrLanes + kWave - 1) / kWave); }
+    // Threads of an update workgroup.  At most one of the granule's BDF
+    // kernel fits on a CU (its channel table takes the LDS).  Four waves, one
+    // per SIMD, while they hold every neuron at once; then eight, whose
+    // shorter Newton iterations beat one neuron per group at a time (20,000
+    // cells: 102 us with 8, 113 us with 16 waves); sixteen once each group
+    // takes four neurons or more (200,000 cells: 495 us with 16, 543 us with
+    // 8; 50,000: 175 and 178 us).
+    int update_threads() const {
+        if (!granule_bdf()) return kBlock;
+        const int w = (granule_waves() + n_cu - 1) / n_cu;
+        return kWave * (w <= 4 ? 4 : (w < 32 ? 8 : 16));
+    }
     // workgroups of the update launch: one per tile, except the granule's
-    // BDF kernel, whose waves take neurons from equal ranges (at most one
-    // workgroup per CU fits)
+    // BDF kernel, whose waves take neurons from equal ranges
     int update_blocks() const {
-        const int t = update_tiles();
-        return (model == EDLUT_GRANULE && integ == EDLUT_BDF && n_cu > 0 && n_cu < t) ? n_cu : t;
+        if (!granule_bdf()) return update_tiles();
+        const int w = update_threads() / kWave;
+        return std::min(n_cu, (granule_waves() + w - 1) / w);
     }
 
     FoldTarget fold_target(int par, bool by_step = false) const {
@@ -1179,7 +1195,7 @@ UpdateFn pick_update(const edlut_population *p, bool ext) {
                                                (int)(sizeof(float) * kGrTable * kGrVars)) == hipSuccess;
             return ok;
         }();
-        if (model == EDLUT_GRANULE && integ == EDLUT_BDF && !lds_ok) return nullptr;
+        if (p->granule_bdf() && !lds_ok) return nullptr;
         const int idx = integ * 2 + (ext ? 1 : 0);
         return model == EDLUT_GRANULE ? gr.fn[idx] : pk.fn[idx];
     }
@@ -1902,7 +1918,7 @@ int edlut_population_update(edlut_population *p, int64_t step, int *n_spikes) {
     if (!fn) return fail(EDLUT_E_ARG, "no update kernel for this model, integrator and synapse set");
     p->started = true;
     const int tiles = p->update_tiles();
-    hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(kBlock), update_lds_bytes(p), p->stream, a);
+    hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), p->stream, a);
     launch_compact(p->stream, p->tile_count, p->staging, tiles, kBlock * p->items, p->spk_idx, p->spk_cnt,
                    1, 0, nullptr, nullptr, nullptr, 0, p->err, StepRef{nullptr, (int32_t)step});
     HIP_TRY(hipGetLastError());
@@ -1996,7 +2012,7 @@ int edlut_population_update_noalloc(edlut_population *p, int64_t step, const int
     a.fold = t;
     p->started = true;
     const int tiles = p->update_tiles();
-    hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(kBlock), update_lds_bytes(p), st, a);
+    hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), st, a);
     launch_compact(st, p->tile_count, p->staging, tiles, kBlock * p->items, spk_idx, spk_cnt, 1, 0, nullptr,
                    nullptr, nullptr, 0, p->err, StepRef{nullptr, (int32_t)step});
     HIP_TRY(hipGetLastError());
@@ -2527,7 +2543,7 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
         a.clk_first = (int32_t)n->clk_first;
         a.clk_count = (int32_t)n->clk_count;
     }
-    hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(kBlock), update_lds_bytes(p), p->stream, a);
+    hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), p->stream, a);
     CompactArgs c = compact_args(n->tile_count, n->staging, tiles, kBlock * p->items, n->own_ring_idx,
                                  n->own_ring_cnt, n->ring, p->n, n->log_cap ? n->log_step : nullptr,
                                  n->log_cap ? n->log_idx : nullptr, n->log_count, n->log_cap, p->err, step);
@@ -3242,7 +3258,8 @@ int edlut_network_set_timing(edlut_network *n, int64_t max_steps) {
     n->clk_cap = 0;
     n->dirty = true;
     if (max_steps == 0) return 0;
-    n->clk_tiles_max = n->pop->stride / kFlagTile;   // the most workgroups of any launch shape
+    // the most workgroups of any launch shape
+    n->clk_tiles_max = std::max<int64_t>(n->pop->stride / kFlagTile, n->pop->update_blocks());
     int rc;
     if ((rc = dalloc(&n->clk, 2 * (size_t)max_steps * (size_t)n->clk_tiles_max)) ||
         (rc = dalloc(&n->clk_next, (size_t)max_steps)))

@@ -485,13 +485,25 @@ __global__ __launch_bounds__(kBlock) void k_update(UpdateArgs a) {
 }
 
 
+// The queued events of neuron i's key of synapse type ty, added to its
+// conductance g in order.
+__device__ __forceinline__ float fold_key(const UpdateArgs &a, int32_t step, int ty, uint32_t i, float g) {
+    const uint64_t key = (uint64_t)ty * (uint64_t)a.stride + (uint64_t)i;
+    if (a.fold.seg_off) {
+        const uint32_t m = a.fold.fill[key];
+        return m >= 1u ? fold_static(a.fold.fill, a.fold.seg_off, a.fold.b_ent, a.fold.rtab, step & 1, key, m, g) : g;
+    }
+    const uint32_t m = a.fold.cnt[key];
+    return m >= 2u ? fold_segment(a.fold.cnt, a.fold.fill, a.fold.seg, a.fold.b_ent, a.fold.b_cap, a.fold.err, key,
+                                  m, g) : g;
+}
+
 // Loads the state of neuron i at the start of a BDF step into sf: the row
 // values, the ordered fold of its multi-event keys when its tile's fold flag
 // is set, and the external drive.
 template <class M, unsigned MASK, bool EXT>
 __device__ __forceinline__ void bdf_load(const UpdateArgs &a, float *__restrict__ const *row, int32_t step,
                                          uint32_t step_key, uint32_t flag, uint32_t i, float *sf) {
-    const int64_t ld = a.stride;
 #pragma unroll
     for (int j = 0; j < M::ND; j++) sf[j] = row[j][i];
     sf[M::EXC] = (MASK & 1u) ? row[M::EXC][i] : 0.0f;
@@ -500,22 +512,8 @@ __device__ __forceinline__ void bdf_load(const UpdateArgs &a, float *__restrict_
     sf[M::EXT] = (MASK & 8u) ? row[M::EXT][i] : 0.0f;
     if (flag) {
 #pragma unroll
-        for (int ty = 0; ty < 3; ty++) {
-            if (!(MASK & (1u << ty))) continue;
-            const uint64_t key = (uint64_t)ty * (uint64_t)ld + (uint64_t)i;
-            if (a.fold.seg_off) {
-                const uint32_t m = a.fold.fill[key];
-                if (m >= 1u)
-                    sf[M::EXC + ty] = fold_static(a.fold.fill, a.fold.seg_off, a.fold.b_ent,
-                                                  a.fold.rtab, step & 1, key, m, sf[M::EXC + ty]);
-                continue;
-            }
-            const uint32_t m = a.fold.cnt[key];
-            if (m >= 2u)
-                sf[M::EXC + ty] = fold_segment(a.fold.cnt, a.fold.fill, a.fold.seg, a.fold.b_ent,
-                                               a.fold.b_cap, a.fold.err, key, m,
-                                               sf[M::EXC + ty]);
-        }
+        for (int ty = 0; ty < 3; ty++)
+            if (MASK & (1u << ty)) sf[M::EXC + ty] = fold_key(a, step, ty, i, sf[M::EXC + ty]);
     }
     if (EXT) {
         const uint32_t u = drive_hash_keyed(step_key, i);
@@ -601,149 +599,6 @@ __global__ __launch_bounds__(kBlock) void k_update_bdf(UpdateArgs a) {
         bdf_store<M, MASK>(a, row, i, out);
     }
     tile_spikes_item_major<ITEMS>(a.out, tile, spk, idx);
-    clock_finish(a, step);
-}
-
-// Granule BDF update (EgidioGranuleCell_TimeDriven with BDFn, the
-// reference's per-neuron step).  The corrector runs a data-dependent number
-// of Newton iterations per neuron (about 3 on average, but 10 for the few
-// percent whose iterate ends in a one-ulp cycle), so a wave that gave each
-// lane a fixed neuron would run each item for its slowest lane's count.
-// Here each wave owns a contiguous range of neurons and a lane takes the
-// range's next neuron as soon as its own corrector has ended; a neuron's
-// arithmetic is the same either way.  The grid is at most one workgroup per
-// CU (the Newton step fills the register file); the ranges are equal.
-//   * The channel table (104 KB) is staged in LDS: every right-hand side
-//     gathers a 26-float row from it.  A lane's first previous-state row
-//     (15 floats) is copied to LDS when it takes a neuron, and the BDF
-//     coefficients are staged there too.
-//   * Spikes set bits of a.bdf.spk_bits; the last workgroup to finish turns
-//     them into the per-tile spike lists (ascending, kFlagTile neurons per
-//     tile) that the compaction reads, clears the bits and the tiles' fold
-//     flags, and resets the workgroup count.
-//   * A lane reads its neuron's fold flag when it takes the neuron.
-constexpr int kGrBatch = 32;
-template <bool EXT>
-__global__ __launch_bounds__(kBlock) void k_update_granule_bdf(UpdateArgs a) {
-    using G = GranuleModel;
-    constexpr unsigned MASK = 15u;   // the synapse types are the run-time mask
-    constexpr int TILE = kFlagTile;
-    const int32_t step = a.step.get();
-    clock_begin(a, step);
-    const int par = a.fold.par_by_step ? (step & 1) : a.fold.par;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        a.fold.bump[par ^ 1] = 0ull;
-        // the next step hands out working-storage slots from the other parity
-        if (a.bdf.ws_count) a.bdf.ws_count[par ^ 1] = 0u;
-    }
-    float *__restrict__ row[G::NV];
-#pragma unroll
-    for (int j = 0; j < G::NV; j++) row[j] = a.state + (int64_t)j * a.stride;
-    const int64_t ld = a.stride;
-    const uint32_t step_key = EXT ? drive_step_key(a.ext.seed, step) : 0u;
-    // each lane's copy of its neuron's first previous-state row, which every
-    // corrector iteration reads (2.4% of the cerebellum step against reading
-    // it from memory once lanes have drifted apart in their range)
-    __shared__ float s_ph0[G::ND * kBlock];
-    // the BDF coefficient table (7 x 7), read by every corrector iteration
-    __shared__ float s_bdfc[49];
-    extern __shared__ float4 s_chan[];
-    {
-        const float4 *g4 = (const float4 *)a.chan;
-        for (int q = threadIdx.x; q < kGrTable * kGrVars / 4; q += kBlock) s_chan[q] = g4[q];
-        if (threadIdx.x < 49) s_bdfc[threadIdx.x] = a.bdf.C[threadIdx.x];
-    }
-    __syncthreads();
-    BdfState bl = a.bdf;
-    bl.C = s_bdfc;
-    RhsCtx c;
-    c.chan = (const float *)s_chan;
-    c.exp_lut = a.exp_lut;
-    c.nmda_lut = a.nmda_lut;
-    c.refr = a.refr;
-    c.refr_len = a.refr_len;
-    c.since_spike = 1 << 30;
-    const float dt = a.k.dt;
-    const int lane = threadIdx.x & (kWave - 1);
-    const uint64_t below = (1ull << lane) - 1ull;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kWavesPerBlock + threadIdx.x / kWave));
-    const int64_t n_waves = (int64_t)gridDim.x * kWavesPerBlock;
-    int cursor = (int)((int64_t)a.n * wave / n_waves);
-    const int end = (int)((int64_t)a.n * (wave + 1) / n_waves);
-    int i = -1;          // neuron on this lane (-1: none)
-    int st = 0, k = 0;
-    float epsi = 1.0f, prev = 0.0f;
-    float S[G::NV], P[G::NV];
-    for (;;) {
-        bool busy = i >= 0 && epsi > 1e-6 && k < 10;   // the corrector's loop condition
-        const uint64_t run = __ballot(busy);
-        // lanes whose corrector has ended wait until kGrBatch lanes are free,
-        // then all commit and take new neurons together
-        if (__popcll(run) <= kWave - kGrBatch) {
-            if (i >= 0 && !busy) {
-                granule_bdf_commit<MASK>(a.mp, a.bdf, ld, (uint32_t)i, st, S, P);
-                const bool fired = G::spike(a.mp, prev, S);
-                a.bdf.st[i] = st;
-                if (fired) {
-                    if (a.last_spike) a.last_spike[i] = step;
-                    atomicOr(&a.bdf.spk_bits[i >> 5], 1u << (i & 31));
-                }
-                bdf_store<G, MASK>(a, row, (uint32_t)i, S);
-                i = -1;
-            }
-            if (cursor < end) {
-                const uint64_t idle = __ballot(i < 0);
-                if (i < 0) {
-                    const int j = cursor + __popcll(idle & below);
-                    if (j < end) {
-                        i = j;
-                        const uint32_t flag = a.fold.tile_flag[j / TILE];
-                        bdf_load<G, MASK, EXT>(a, row, step, step_key, flag, (uint32_t)i, S);
-                        prev = S[0];
-                        st = a.bdf.st[i];
-                        if (a.last_spike) c.since_spike = step - 1 - a.last_spike[i];
-                        granule_bdf_predict<MASK>(a.mp, c, dt, a.bdf, ld, (uint32_t)i, st, S, P);
-                        if (st > 1) {
-                            const float *Ph = (const float *)a.bdf.prev;
-#pragma unroll
-                            for (int q = 0; q < G::ND; q++) s_ph0[q * kBlock + threadIdx.x] = Ph[(int64_t)q * ld + i];
-                        }
-                        epsi = 1.0f;
-                        k = 0;
-                        busy = true;
-                    }
-                }
-                cursor += __popcll(idle);
-            }
-        }
-        if (!__any(busy)) break;
-        if (busy)
-            granule_bdf_newton<MASK>(a.mp, c, dt, bl, par, ld, (uint32_t)i, st, S, P, epsi, k, s_ph0 + threadIdx.x);
-    }
-    __shared__ uint32_t s_last;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        __threadfence();
-        s_last = atomicAdd(a.bdf.done, 1u) == gridDim.x - 1u;
-    }
-    __syncthreads();
-    if (s_last) {
-        __threadfence();
-        for (int t = threadIdx.x; t < a.n_tiles; t += kBlock) {
-            int32_t cnt = 0;
-            for (int w = 0; w < TILE / 32; w++) {
-                uint32_t bits = atomicExch(&a.bdf.spk_bits[t * (TILE / 32) + w], 0u);
-                while (bits) {
-                    const int b = __builtin_ctz(bits);
-                    bits &= bits - 1u;
-                    a.out.staging[(int64_t)t * TILE + cnt++] = t * TILE + w * 32 + b;
-                }
-            }
-            a.out.tile_count[t] = cnt;
-            clear_tile_flag<TILE>(a.fold.tile_flag, t);
-        }
-        if (threadIdx.x == 0) *a.bdf.done = 0u;
-    }
     clock_finish(a, step);
 }
 
