@@ -573,6 +573,7 @@ struct EqSim {
     EqItem *heap = nullptr;
     int32_t *st = nullptr;
     int32_t cap = 0;
+    int64_t in_flight = 0;          // heap entries when every update queues one group per delay
     uint32_t *err = nullptr;
     int64_t next_first = 1;
     double h_pop = 0.0;
@@ -831,6 +832,19 @@ int eq_build(EqSim *S, const std::vector<edlut_network *> &nets, uint32_t *err, 
     }
     if (cap > (1ll << 28)) return fail(EDLUT_E_CAP, "event queue too large");
     S->cap = (int32_t)cap;
+    // a group of delay d waits d updates; the update and stop events, and the
+    // groups the window being replayed adds before it removes any
+    S->in_flight = 2 * (int64_t)S->em.size() + 2;
+    for (EqHostEm &E : S->em) {
+        if (E.kind == kEqTrain) {
+            const Source &s0 = E.copies[0].first->sources[(size_t)E.copies[0].second];
+            S->in_flight += (int64_t)s0.tr_t.size();
+            continue;
+        }
+        S->in_flight += D;
+        for (int d = 1; d <= D; d++)
+            if ((E.dev.full[(d - 1) >> 5] >> ((d - 1) & 31)) & 1u) S->in_flight += d + 1;
+    }
     if ((rc = dalloc(&S->heap, (size_t)cap + 1)) || (rc = dalloc(&S->st, kEqSt + S->em.size())) ||
         (rc = dalloc(&S->d_em, S->em.size())))
         return rc;
@@ -1345,14 +1359,20 @@ RingFoldFn pick_ring_fold(int pass, int lanes) {
     }
 }
 using CompactFoldEqFn = void (*)(CompactArgs, FoldTarget, RingEvents, int, EqArgs);
-CompactFoldEqFn pick_compact_fold_eq(int lanes) {
+template <int ITEMS>
+CompactFoldEqFn compact_fold_eq_fn(int lanes) {
     switch (lanes) {
-        case 8: return k_compact_fold_eq<8>;
-        case 16: return k_compact_fold_eq<16>;
-        case 32: return k_compact_fold_eq<32>;
-        case 64: return k_compact_fold_eq<64>;
+        case 8: return k_compact_fold_eq<8, ITEMS>;
+        case 16: return k_compact_fold_eq<16, ITEMS>;
+        case 32: return k_compact_fold_eq<32, ITEMS>;
+        case 64: return k_compact_fold_eq<64, ITEMS>;
         default: return nullptr;
     }
+}
+// By fold lanes and the heap entries the replay keeps in LDS.
+CompactFoldEqFn pick_compact_fold_eq(int lanes, const EqSim *eq) {
+    return eq->in_flight <= kEqFusedItems ? compact_fold_eq_fn<kEqFusedItems>(lanes)
+                                          : compact_fold_eq_fn<kEqItems>(lanes);
 }
 using CompactFoldFn = void (*)(CompactArgs, FoldTarget, RingEvents, int);
 CompactFoldFn pick_compact_fold(int lanes) {
@@ -2563,7 +2583,7 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
         RingEvents rn = re0;
         rn.step = StepRef{step.ptr, step.imm + 1};
         if (eq_fused) {
-            CompactFoldEqFn f = pick_compact_fold_eq(n->fold_lanes);
+            CompactFoldEqFn f = pick_compact_fold_eq(n->fold_lanes, eq);
             if (!f) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
             hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks + 1), dim3(kBlock), 0, p->stream, c, ft, rn, nbc,
                                eq_args(eq, step, 0, 0.0));

@@ -33,7 +33,6 @@ enum EqEmitterKind : int { kEqPop = 0, kEqPoisson = 1, kEqTrain = 2 };
 constexpr int kEqMaxEmitters = 16;
 constexpr int kEqMaskWords = 8;          // delays up to 256 steps
 constexpr int kEqChunk = 1024;           // PropagatedSpikeGroup::MaxSize
-constexpr int kEqLdsItems = 2048;        // heap entries staged in LDS (larger heaps stay in memory)
 
 // Heap entry: time, then a = priority<<28 | kind<<24 | emitter<<16 | d (or j),
 // b = chunk (groups) or input record (input and propagated spikes).
@@ -183,17 +182,26 @@ constexpr int kMaxDelayEq = 32 * kEqMaskWords;
 // The heap operations of one window, run by one wave with wave-uniform
 // control flow (always inlined, so that a heap staged in LDS is addressed as
 // LDS).  Each heap operation is the reference's, lane-parallel:
-//  - removal: every lane takes one node p of the top 64 and picks its child
-//    as the reference's sift-down would (the earlier child, the left one on
-//    ties), and whether that child moves up past the displaced last element;
-//    the path is then a chain of readlanes from the root, and the nodes on
-//    it take their chosen child's entry in one write.  Nodes below the top
-//    64 (heaps of more than 129 entries) continue one level at a time.
+//  - removal: every lane takes one of the 63 nodes of the top six levels,
+//    picks its child as the reference's sift-down would (the earlier child,
+//    the left one on ties), and whether that child moves up past the
+//    displaced last element.  Two ballots of those bits, compared under the
+//    lane's constant masks of its ancestors, tell whether its node is on the
+//    path; the nodes on it take their chosen child's entry, and the last one
+//    the displaced element, in one write.  A path that leaves the six levels
+//    goes on in the next six, from the child it leaves through.
 //  - insertion: lane j reads the j-th ancestor of the new position; the
 //    ancestors later than the new entry up to the first that is not (the
 //    reference's sift-up stops there) move down one level in one write.
-// Children of node p are read before any entry on the path is written, as in
+// Children of a node are read before any entry on the path is written, as in
 // the reference, where the entries written lie above them.
+//
+// Bound by the latency of one wave's instruction chain (about 7 cycles each).
+// The launch that holds the replay, with a chain of 12 tests per lane and
+// insertions one by one, then with the ancestor masks and batched insertions:
+// 14.5 us and 11.3 us (1M AdEx cells, 10 delays, 57 entries), 79.7 us and
+// 41.1 us (125,000 Poisson sources, 41 delays, 1,250 entries; in memory, then
+// in LDS).
 struct EqWin {
     int32_t n;          // heap size
     uint32_t r;         // rank counter of the window
@@ -227,105 +235,139 @@ __device__ __forceinline__ EqItem eq_lane0(const EqItem &v) {
     return r;
 }
 
-// Inserts x; `top` follows the heap's first entry.
-__device__ __forceinline__ void eq_insert_wave(EqItem *__restrict__ h, int32_t &n, const EqItem &x, EqItem &top) {
+// A ballot of a condition the compiler holds as a lane mask.
+__device__ __forceinline__ uint64_t eq_ballot(bool x) { return __builtin_amdgcn_ballot_w64(x); }
+
+// Inserts x at position c, the first free one of a heap that holds every
+// entry before it; `top` follows the heap's first entry.
+__device__ __forceinline__ void eq_insert_at(EqItem *__restrict__ h, int32_t c, const EqItem &x, EqItem &top) {
     const int lane = eq_lane();
-    const int32_t c = ++n;
     const int depth = 31 - __builtin_clz((uint32_t)c);     // ancestors of c
     // lanes past the root read entry 0 (unused) and take no part
     const EqItem anc = h[lane < depth ? c >> (lane + 1) : 0];
-    const bool later = (lane < depth) & eq_later_v(anc, x);
-    const uint64_t lm = __ballot(later);
+    const uint64_t lm = eq_ballot((lane < depth) & eq_later_v(anc, x));
     const int m = (int)__builtin_ctzll(~lm);                // ancestors that move down
-    if (lane < m) h[c >> lane] = anc;
-    if (lane == 0) h[c >> m] = x;
+    EqItem v;
+    v.t = lane < m ? anc.t : x.t;
+    v.a = lane < m ? anc.a : x.a;
+    v.b = lane < m ? anc.b : x.b;
+    if (lane <= m) h[c >> lane] = v;
     if ((c >> m) == 1) top = x;
 }
 
-// The entries a removal reads (the last entry and the children of the top
-// 64 nodes), loaded before the caller decides to remove.
-struct EqRemoveLoads {
-    EqItem x, ch;
-    int32_t c;
-    bool has_l;
-};
+// Inserts the entries x of the lanes in `bits`, ascending lanes first.  An
+// entry that is no earlier than its parent stays where it is put; insertions
+// before it can only make the parent earlier.  Those entries are written
+// together; the others (and those whose parent is itself one of the batch)
+// follow one by one at the places they would have had.
+__device__ __forceinline__ void eq_insert_batch(EqItem *__restrict__ h, int32_t &n, uint64_t bits, const EqItem &x,
+                                                EqItem &top) {
+    const int lane = eq_lane();
+    const bool mine = (bits >> lane) & 1ull;
+    const int32_t c = n + 1 + (int32_t)__popcll(bits & ((1ull << lane) - 1ull));
+    const bool inside = mine & (c / 2 <= n) & (c > 1);
+    const EqItem parent = h[inside ? c / 2 : 0];
+    const bool stays = inside & !eq_later_v(parent, x);
+    if (stays) h[c] = x;
+    n += (int32_t)__popcll(bits);
+    uint64_t rest = eq_ballot(mine & !stays);
+    const uint64_t tb = (uint64_t)__double_as_longlong(x.t);
+    while (rest) {
+        const int b = __builtin_ctzll(rest);
+        rest &= rest - 1ull;
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)tb, b);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(tb >> 32), b);
+        EqItem y;
+        y.t = __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+        y.a = (uint32_t)__builtin_amdgcn_readlane((int)x.a, b);
+        y.b = (uint32_t)__builtin_amdgcn_readlane((int)x.b, b);
+        eq_insert_at(h, __builtin_amdgcn_readlane(c, b), y, top);
+    }
+}
 
-__device__ __forceinline__ EqRemoveLoads eq_remove_loads(const EqItem *__restrict__ h, int32_t n) {
-    const int32_t p0 = eq_lane() + 1;
+// A lane's node in a block of six levels (node lane + 1 of the block, counted
+// from its root; lane 63 has none), and its ancestors there (nodes 1 to 31,
+// bit q - 1 for node q) by the direction the path must take at them.
+struct EqNode {
+    int level, off;
+    uint32_t left, right;
+};
+__device__ __forceinline__ EqNode eq_node() {
+    const uint32_t r = (uint32_t)eq_lane() + 1u;
+    EqNode q;
+    q.level = 31 - __builtin_clz(r);
+    q.off = (int)(r - (1u << q.level));
+    q.left = q.right = 0u;
+#pragma unroll
+    for (int j = 1; j <= 5; j++) {
+        if ((r >> j) == 0u) continue;
+        const uint32_t bit = 1u << ((r >> j) - 1u);
+        if ((r >> (j - 1)) & 1u) q.right |= bit;
+        else q.left |= bit;
+    }
+    return q;
+}
+
+// What a removal reads of the block rooted at p: the last entry x and the
+// children of the lane's node (indices clamped into the heap), loaded before
+// the caller decides to remove.
+struct EqRemoveLoads {
+    EqItem x, L, R;
+};
+__device__ __forceinline__ EqRemoveLoads eq_remove_loads(const EqItem *__restrict__ h, int32_t n, int32_t p,
+                                                         const EqNode &q) {
     const int32_t size = n - 1 > 0 ? n - 1 : 1;
-    // both children of node p0, read unconditionally (indices clamped into
-    // the heap), then chosen with selects
-    const int32_t cl = 2 * p0, cr = 2 * p0 + 1;
-    const EqItem L = h[cl <= size ? cl : size];
-    const EqItem R = h[cr <= size ? cr : size];
-    const bool has_r = cr <= n - 1;
-    const bool pick_r = has_r & eq_later_v(L, R);
+    const int32_t cl = 2 * ((p << q.level) + q.off);
     EqRemoveLoads r;
+    r.L = h[cl <= size ? cl : size];
+    r.R = h[cl < size ? cl + 1 : size];
     r.x = h[n];
-    r.ch.t = pick_r ? R.t : L.t;
-    r.ch.a = pick_r ? R.a : L.a;
-    r.ch.b = pick_r ? R.b : L.b;
-    r.c = pick_r ? cr : cl;
-    r.has_l = cl <= n - 1;
     return r;
 }
 
-// Removes the top (n >= 1) with the entries `eq_remove_loads` read; `top`
-// becomes the new first entry.  Two ballots give, for each of the top 64
-// nodes, whether its chosen child moves up and whether that child is the
-// right one; every lane then tests its node's ancestors against those bits,
-// so the path comes out without a chain of dependent steps.
-__device__ __forceinline__ void eq_remove_wave(EqItem *__restrict__ h, int32_t &n, const EqRemoveLoads &r,
+// Removes the top (n >= 1) with the entries `eq_remove_loads` read of the
+// top block; `top` becomes the new first entry.
+__device__ __forceinline__ void eq_remove_wave(EqItem *__restrict__ h, int32_t &n, EqRemoveLoads r, const EqNode &q,
                                                EqItem &top) {
-    const int lane = eq_lane();
     if (n == 1) {
         n = 0;
         return;
     }
+    const int lane = eq_lane();
     const int32_t size = --n;
-    const bool ok = r.has_l & eq_before_v(r.ch, r.x);
-    const uint64_t moves = __ballot(ok);
-    const uint64_t right = __ballot((r.c & 1) != 0);
-    // node p0 (lane + 1) is on the path when every ancestor moves its child
-    // up and chose the child toward p0
-    const uint32_t p0 = (uint32_t)lane + 1u;
-    bool on = true;
-#pragma unroll
-    for (int j = 1; j <= 6; j++) {
-        const uint32_t q = p0 >> j;          // ancestor j levels up (0: none)
-        const uint32_t sh = (q - 1u) & 63u;
-        const bool step = (q == 0u) | ((((moves >> sh) & 1ull) != 0ull) &
-                                       ((uint32_t)((right >> sh) & 1ull) == ((p0 >> (j - 1)) & 1u)));
-        on = on & step;
-    }
-    const uint64_t path = __ballot(on & ok);
-    const uint64_t ends = __ballot(on & !ok);
-    int32_t p;
-    if (ends) {
-        p = (int32_t)__builtin_ctzll(ends) + 1;
-    } else {
-        // the path leaves the top 64 nodes below its deepest node there
-        const uint64_t out = __ballot(on & ok & (r.c > 64));
-        p = __builtin_amdgcn_readlane(r.c, (int)__builtin_ctzll(out));
-    }
-    if ((path >> lane) & 1ull) h[lane + 1] = r.ch;
-    top = (moves & 1ull) ? eq_lane0(r.ch) : r.x;
-    // below the top 64 nodes: one level at a time
-    while (p > 64 && 2 * p <= size) {
-        int32_t cc = 2 * p;
-        EqItem a = h[cc];
-        if (cc + 1 <= size) {
-            const EqItem b = h[cc + 1];
-            if (eq_later(a, b)) {
-                a = b;
-                cc++;
-            }
+    const EqItem x = r.x;
+    int32_t p = 1;
+    for (;;) {
+        const int32_t node = (p << q.level) + q.off, cl = 2 * node;
+        const bool pick_r = (cl < size) & eq_later_v(r.L, r.R);
+        EqItem ch;
+        ch.t = pick_r ? r.R.t : r.L.t;
+        ch.a = pick_r ? r.R.a : r.L.a;
+        ch.b = pick_r ? r.R.b : r.L.b;
+        const bool ok = (lane < 63) & (cl <= size) & eq_before_v(ch, x);
+        // nodes 1 to 31 whose child does not move up to the left / right
+        const uint32_t moves = (uint32_t)eq_ballot(ok), right = (uint32_t)eq_ballot(pick_r);
+        const uint32_t no_r = ~(moves & right), no_l = ~(moves & ~right);
+        const bool on = (lane < 63) & (((q.right & no_r) | (q.left & no_l)) == 0u);
+        EqItem v;
+        v.t = ok ? ch.t : x.t;
+        v.a = ok ? ch.a : x.a;
+        v.b = ok ? ch.b : x.b;
+        if (on) h[node] = v;
+        if (p == 1) top = eq_lane0(v);
+        // the path ends at the node that takes x, or leaves through the last level
+        if (eq_ballot(on & !ok)) break;
+        const uint64_t out = eq_ballot(on & (q.level == 5));
+        const int from = (int)__builtin_ctzll(out);
+        p = __builtin_amdgcn_readlane(cl + (pick_r ? 1 : 0), from);
+        if (2 * p > size) {
+            if (lane == 0) h[p] = x;
+            break;
         }
-        if (!eq_before(a, r.x)) break;
-        if (lane == 0) h[p] = a;
-        p = cc;
+        const int32_t c2 = 2 * ((p << q.level) + q.off);
+        r.L = h[c2 <= size ? c2 : size];
+        r.R = h[c2 < size ? c2 + 1 : size];
     }
-    if (lane == 0) h[p] = r.x;
 }
 
 // Ranks given in a window, listed in LDS and written to the models' rank
@@ -340,7 +382,7 @@ __device__ __forceinline__ void eq_window(EqItem *__restrict__ h, const EqArgs &
                                           const double *delay_s, uint4 *rk, int32_t k, EqWin &w) {
     const int lane = eq_lane();
     const int par = (k + 1) & 1;          // parity of the update that consumes this window
-    EqItem top = h[1];                    // the heap's first entry, kept in registers
+    EqItem top = eq_lane0(h[1]);          // the heap's first entry, kept in registers
     int32_t nrk = 0;
     auto flush = [&]() {
         for (int i = lane; i < nrk; i += 64) {
@@ -362,7 +404,7 @@ __device__ __forceinline__ void eq_window(EqItem *__restrict__ h, const EqArgs &
             w.overflow = true;
             return;
         }
-        eq_insert_wave(h, w.n, x, top);
+        eq_insert_at(h, ++w.n, x, top);
     };
     if (a.resume) {
         // input spikes added since the last run (Simulation_API::
@@ -389,16 +431,17 @@ __device__ __forceinline__ void eq_window(EqItem *__restrict__ h, const EqArgs &
         }
         if (a.with_stop) push(eq_item(a.stop_t, kEqPrioStop, kEqStop, 0, 0, 0));
     }
+    const EqNode node = eq_node();
     uint32_t pops = 0;                    // models that are populations
     for (int e = 0; e < a.n_em; e++) pops |= (em[e].kind == kEqPop ? 1u : 0u) << e;
     while (w.n > 0 && !w.overflow) {
         const EqItem it = top;
-        const EqRemoveLoads rl = eq_remove_loads(h, w.n);
+        const EqRemoveLoads rl = eq_remove_loads(h, w.n, 1, node);
         const uint32_t top_a = __builtin_amdgcn_readfirstlane(it.a);
         const uint32_t kind = (top_a >> 24) & 0xfu, e = (top_a >> 16) & 0xffu;
         // the window ends where the populations' next update starts
         if (kind == kEqTime && ((pops >> e) & 1u) && next_k[e] > k) break;
-        eq_remove_wave(h, w.n, rl, top);
+        eq_remove_wave(h, w.n, rl, node, top);
         if (kind == kEqStop) {
             w.stop_r = (int32_t)w.r;
             break;
@@ -437,24 +480,21 @@ __device__ __forceinline__ void eq_window(EqItem *__restrict__ h, const EqArgs &
                 if (lane == 0) cur[bd - 1] = cb + 1u;
             }
             // the partial groups: delays whose count is not a multiple of
-            // 1,024, 64 delays at a time (lane L holds the time of delay L + 1)
+            // 1,024, 64 delays at a time (lane L holds the group of delay L + 1)
             for (int j = 0; j * 64 < a.max_delay; j++) {
                 uint64_t bits = (uint64_t)pmask[e][2 * j];
                 if (2 * j + 1 < MAXD / 32 + 1) bits |= (uint64_t)pmask[e][2 * j + 1] << 32;
                 if (!bits) continue;
                 const int dl = j * 64 + lane + 1;
-                const uint64_t tb = (uint64_t)__double_as_longlong(it.t + delay_s[dl <= a.max_delay ? dl : 0]);
-                while (bits) {
-                    const int b = __builtin_ctzll(bits);
-                    bits &= bits - 1ull;
-                    const int d = j * 64 + b + 1;
-                    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)tb, b);
-                    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(tb >> 32), b);
-                    const double td = __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-                    uint32_t ch = 0u;
-                    if (any_full) ch = cur[d - 1];
-                    push(eq_item(td, kEqPrioSpike, kEqGroup, e, (uint32_t)d, ch));
+                EqItem x;
+                x.t = it.t + delay_s[dl <= a.max_delay ? dl : 0];
+                x.a = eq_item(0.0, kEqPrioSpike, kEqGroup, e, (uint32_t)dl, 0u).a;
+                x.b = any_full ? cur[(dl - 1) % MAXD] : 0u;
+                if (w.n + (int32_t)__popcll(bits) > a.cap) {
+                    w.overflow = true;
+                    break;
                 }
+                eq_insert_batch(h, w.n, bits, x, top);
             }
             if (lane == 0) next_k[e] = ke + 1;
             push(eq_item(it.t + E.h, kEqPrioTime, kEqTime, e, 0, 0));
@@ -500,7 +540,7 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
     __shared__ int32_t s_scan[kBlock], s_scan2[kBlock];
     __shared__ int32_t s_run, s_base;
     __shared__ int32_t s_st[kEqSt];
-    __shared__ int32_t s_in_lds;
+    __shared__ int32_t s_groups;
     __shared__ double s_delay[MAXD + 1];
     __shared__ uint32_t s_pmask[kEqMaxEmitters][MAXD / 32 + 1];
     __shared__ uint32_t s_anyfull[kEqMaxEmitters];
@@ -520,8 +560,9 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
         s_next[threadIdx.x] = a.st[kEqSt + threadIdx.x];
     }
     for (int d = threadIdx.x; d <= a.max_delay; d += kBlock) s_delay[d] = a.delay_s[d];
-    for (int i = threadIdx.x; i < kEqMaxEmitters * MAXD; i += kBlock) (&s_cnt[0][0])[i] = 0u;
+    for (int i = threadIdx.x; i < a.n_em * MAXD; i += kBlock) (&s_cnt[0][0])[i] = 0u;
     if (threadIdx.x < kEqMaxEmitters) s_partial[threadIdx.x] = 0u;
+    if (threadIdx.x == 0) s_groups = 0;
     __syncthreads();
     const int32_t size0 = s_st[0];
     // stage the heap in LDS speculatively (the check below may discard it)
@@ -554,15 +595,9 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
             }
 #pragma unroll
             for (int off = 32; off > 0; off >>= 1) tot += __shfl_xor(tot, off);
-            if ((threadIdx.x & 63u) == 0 && tot > 0)
-                for (int w = 0; w < a.words; w++) {
-                    uint32_t bits = E.full[w];
-                    while (bits) {
-                        const int b = __builtin_ctz(bits);
-                        bits &= bits - 1u;
-                        atomicAdd(&s_cnt[e][(w * 32 + b) % MAXD], (uint32_t)tot);
-                    }
-                }
+            // lane d adds the wave's spikes to delay d + 1
+            for (int d = eq_lane(); d < a.max_delay && tot > 0; d += 64)
+                if ((E.full[d >> 5] >> (d & 31)) & 1u) atomicAdd(&s_cnt[e][d % MAXD], (uint32_t)tot);
             continue;
         }
         auto count = [&](int32_t id) {
@@ -601,23 +636,33 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
         }
     }
     __syncthreads();
-    // per model (one wave each): delays with a partial group, and whether
-    // any group is full, from ballots over 64 delays at a time
-    for (int e = (int)(threadIdx.x >> 6); e < kEqMaxEmitters; e += kBlock / 64) {
+    // per model (one wave each): delays with a partial group, whether any
+    // group is full, and the groups the update can queue
+    for (int e = (int)(threadIdx.x >> 6); e < a.n_em; e += kBlock / 64) {
         const int lane = eq_lane();
         bool full = false;
+        int32_t groups = a.max_delay;
 #pragma unroll
         for (int j = 0; j < (MAXD + 63) / 64; j++) {
             const int d = j * 64 + lane + 1;
             const uint32_t c = d <= MAXD && d <= a.max_delay ? s_cnt[e][(d - 1) % MAXD] : 0u;
             const uint64_t pm = __ballot((c % (uint32_t)kEqChunk) != 0u);
-            full = full || __ballot(c >= (uint32_t)kEqChunk) != 0ull;
+            if (__ballot(c >= (uint32_t)kEqChunk) != 0ull) {
+                full = true;
+                int32_t g = (int32_t)(c / (uint32_t)kEqChunk);
+                for (int off = 32; off > 0; off >>= 1) g += __shfl_xor(g, off);
+                groups += g;
+            }
             if (lane == 0) {
                 if (2 * j < MAXD / 32 + 1) s_pmask[e][2 * j] = (uint32_t)pm;
                 if (2 * j + 1 < MAXD / 32 + 1) s_pmask[e][2 * j + 1] = (uint32_t)(pm >> 32);
             }
         }
-        if (lane == 0) s_anyfull[e] = full ? 1u : 0u;
+        if (lane == 0) {
+            s_anyfull[e] = full ? 1u : 0u;
+            const EqEmitter &E = s_em[e];
+            atomicAdd(&s_groups, E.kind != kEqTrain ? groups : (a.resume ? E.in_hi - E.in_lo : 0));
+        }
     }
     // 2. last member of every full chunk where a delay has 1,024 spikes or
     // more and not every spiking neuron has every delay (else chunk c ends at
@@ -695,7 +740,6 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
     }
     // 3. the window's rank table is cleared first when the run stops inside
     // it (explicit stop time): groups still queued at the stop hold no rank
-    if (threadIdx.x == 0 && a.resume) s_st[3] = a.clear_step;
     __syncthreads();
     if (!a.resume && s_st[3] == k) {
         const int par = (k + 1) & 1;
@@ -706,20 +750,7 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
         }
     }
     // 4. the heap stays in LDS when it cannot outgrow it in this call
-    if (threadIdx.x == 0) {
-        int64_t bound = (int64_t)size0 + a.n_em + 2;
-        for (int e = 0; e < a.n_em; e++) {
-            const EqEmitter &E = s_em[e];
-            if (E.kind == kEqTrain) {
-                if (a.resume) bound += E.in_hi - E.in_lo;
-                continue;
-            }
-            for (int d = 1; d <= a.max_delay; d++) bound += s_cnt[e][d - 1] / kEqChunk + 1;
-        }
-        s_in_lds = bound <= LDS_ITEMS ? 1 : 0;
-    }
-    __syncthreads();
-    const bool in_lds = s_in_lds != 0;
+    const bool in_lds = (int64_t)size0 + a.n_em + 2 + s_groups <= LDS_ITEMS;
     // 5. the heap operations, by the first wave
     if (threadIdx.x < 64) {
         EqWin w{size0, (uint32_t)s_st[1], -1, false, false};
@@ -741,12 +772,15 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
         for (int i = threadIdx.x; i <= s_st[0]; i += kBlock) a.heap[i] = s_heap[i];
 }
 
-// The replay as a kernel of its own (circuits, plastic networks, resuming calls).
-__global__ __launch_bounds__(kBlock) void k_eventq(EqArgs a) { eq_body<2048, kMaxDelayEq>(a); }
-
-// Sizes of the replay fused into a network's compaction kernel.
+// Heap entries staged in LDS (larger heaps stay in memory).  The replay fused
+// into a network's compaction kernel shares its LDS budget with the fold's
+// workgroups: 16 KB when the network's groups in flight fit, else 64 KB.
+constexpr int kEqItems = 4096;
 constexpr int kEqFusedItems = 1024;
 constexpr int kEqFusedDelays = 64;
+
+// The replay as a kernel of its own (circuits, plastic networks, resuming calls).
+__global__ __launch_bounds__(kBlock) void k_eventq(EqArgs a) { eq_body<kEqItems, kMaxDelayEq>(a); }
 
 }  // namespace edl
 

@@ -874,12 +874,12 @@ __global__ __launch_bounds__(kBlock) void k_compact_fold(CompactArgs c, FoldTarg
 // workgroup (its chain of dependent steps is the longest): it reads update
 // k's spikes from the update kernel's tiles, so it depends on nothing the
 // other workgroups write and runs beside them.
-template <int LANES>
+template <int LANES, int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_compact_fold_eq(CompactArgs c, FoldTarget t, RingEvents r,
                                                             int nb_compact, EqArgs q) {
     clock_next_kernel(c);
     const int b = (int)blockIdx.x - 1;
-    if (b < 0) eq_body<kEqFusedItems, kEqFusedDelays>(q);
+    if (b < 0) eq_body<ITEMS, kEqFusedDelays>(q);
     else if (b < nb_compact) compact_body(c, b, nb_compact);
     else fold_ring_body<kStatic, LANES>(t, r, b - nb_compact, (int)gridDim.x - 1 - nb_compact);
 }
