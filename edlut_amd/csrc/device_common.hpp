@@ -48,10 +48,11 @@ __device__ __forceinline__ int tile_neuron(int tile, int j) {
     return tile * kBlock * ITEMS + wid * ITEMS * kWave + j * kWave + lane;
 }
 
-template <int ITEMS>
+template <int ITEMS, int BLOCK = kBlock>
 __device__ __forceinline__ void tile_spikes(const TileOut &o, int tile, const bool *spike,
                                             const int *idx) {
-    __shared__ uint32_t s_wave[ITEMS * kWavesPerBlock];
+    constexpr int kWaves = BLOCK / kWave;
+    __shared__ uint32_t s_wave[ITEMS * kWaves];
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = threadIdx.x / kWave;
     uint64_t ballot[ITEMS];
@@ -63,46 +64,14 @@ __device__ __forceinline__ void tile_spikes(const TileOut &o, int tile, const bo
     __syncthreads();
     uint32_t local = 0;
 #pragma unroll
-    for (int q = 0; q < ITEMS * kWavesPerBlock; q++) local += s_wave[q];
+    for (int q = 0; q < ITEMS * kWaves; q++) local += s_wave[q];
 #pragma unroll
     for (int j = 0; j < ITEMS; j++) {
         if (spike[j]) {
             uint32_t base = 0;
             for (int q = 0; q < wid * ITEMS + j; q++) base += s_wave[q];
             const uint32_t rank = (uint32_t)__popcll(ballot[j] & ((1ull << lane) - 1ull));
-            o.staging[(int64_t)tile * kBlock * ITEMS + base + rank] = idx[j];
-        }
-    }
-    if (threadIdx.x == 0) o.tile_count[tile] = (int32_t)local;
-}
-
-// The same output for the item-major layout of the BDF kernels (item j of
-// thread t of tile `tile` is neuron tile*kBlock*ITEMS + j*kBlock + t), whose
-// ascending order is item, then wave, then lane: a population smaller than
-// a workgroup gets one neuron per thread.
-template <int ITEMS>
-__device__ __forceinline__ void tile_spikes_item_major(const TileOut &o, int tile, const bool *spike,
-                                                       const int *idx) {
-    __shared__ uint32_t s_wave[ITEMS * kWavesPerBlock];
-    const int lane = threadIdx.x & (kWave - 1);
-    const int wid = threadIdx.x / kWave;
-    uint64_t ballot[ITEMS];
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        ballot[j] = __ballot(spike[j]);
-        if (lane == 0) s_wave[j * kWavesPerBlock + wid] = (uint32_t)__popcll(ballot[j]);
-    }
-    __syncthreads();
-    uint32_t local = 0;
-#pragma unroll
-    for (int q = 0; q < ITEMS * kWavesPerBlock; q++) local += s_wave[q];
-#pragma unroll
-    for (int j = 0; j < ITEMS; j++) {
-        if (spike[j]) {
-            uint32_t base = 0;
-            for (int q = 0; q < j * kWavesPerBlock + wid; q++) base += s_wave[q];
-            const uint32_t rank = (uint32_t)__popcll(ballot[j] & ((1ull << lane) - 1ull));
-            o.staging[(int64_t)tile * kBlock * ITEMS + base + rank] = idx[j];
+            o.staging[(int64_t)tile * BLOCK * ITEMS + base + rank] = idx[j];
         }
     }
     if (threadIdx.x == 0) o.tile_count[tile] = (int32_t)local;
@@ -127,6 +96,12 @@ struct CompactArgs {
     int64_t log_cap;
     uint32_t *err;         // bit 1: log overflow
     StepRef step;
+    // plug-in updates: pinned host memory that takes the total, the error word
+    // and the first host_cap indices (null: none), so that a step with few
+    // spikes needs no copy back
+    int32_t *host_cnt;
+    int32_t *host_idx;
+    int32_t host_cap;
     // timed runs: the earliest workgroup start of this launch, per step in
     // [clk_first, clk_first + clk_count), on the device wall clock (null:
     // untimed).  It ends the previous update kernel's launch as a kernel
@@ -196,6 +171,7 @@ __device__ __forceinline__ void compact_body(const CompactArgs &a, int bid, int 
         for (int j = 0; j < c; j++) {
             const int32_t id = a.staging[(int64_t)t * a.tile_size + j];
             out_idx[start + j] = id;
+            if (a.host_idx && start + j < a.host_cap) a.host_idx[start + j] = id;
             if (a.log_idx) {
                 const int64_t lp = log_base + start + j;
                 if (lp < a.log_cap) {
@@ -208,6 +184,10 @@ __device__ __forceinline__ void compact_body(const CompactArgs &a, int bid, int 
     if (bid == nb - 1 && threadIdx.x == 0) {
         const int64_t total = base + s_scan[kBlock - 1];
         a.out_count[slot] = (int32_t)total;
+        if (a.host_cnt) {
+            a.host_cnt[0] = (int32_t)total;
+            a.host_cnt[1] = (int32_t)*a.err;
+        }
         if (a.log_count) {
             const int64_t nl = log_base + total;
             if (a.log_idx && nl > a.log_cap) atomicOr(a.err, 2u);

@@ -308,24 +308,24 @@ struct edlut_population {
     int32_t *staging = nullptr;
     int32_t *spk_idx = nullptr;
     int32_t *spk_cnt = nullptr;
-    int32_t *h_spk = nullptr;   // pinned
-    int32_t *h_cnt = nullptr;   // pinned
+    int32_t *h_spk = nullptr;   // pinned: the last update's spikes
+    int32_t *h_cnt = nullptr;   // pinned: [2] their number, the error word
     int last_n_spikes = 0;
     uint32_t *err = nullptr;
 
     // ordered input fold
-    uint32_t *cnt = nullptr, *fill = nullptr, *tile_flag = nullptr;
-    uint64_t *seg = nullptr, *bump = nullptr;
-    uint64_t upd_seq = 0;   // plug-in mode: parity of the fold counters
+    uint32_t *fill = nullptr, *tile_flag = nullptr;
+    uint64_t upd_seq = 0;   // plug-in mode: parity of the BDF working storage
     FoldEntry *b_ent = nullptr;
     uint64_t b_cap = 0;
-    std::vector<int32_t> q_tgt;
-    std::vector<uint8_t> q_type;
-    std::vector<float> q_w;
-    int32_t *e_tgt = nullptr;
-    uint8_t *e_type = nullptr;
-    float *e_w = nullptr;
-    int e_cap = 0;
+    // plug-in mode: the step's queued events in pinned memory, which the fold
+    // reads over the bus (targets, weights, types), and their list nodes
+    uint32_t *head = nullptr;
+    FoldNode *node = nullptr;
+    int32_t *q_tgt = nullptr;
+    float *q_w = nullptr;
+    uint8_t *q_type = nullptr;
+    int q_n = 0, q_cap = 0;
 
     edlut_network *net = nullptr;
 
@@ -337,7 +337,10 @@ struct edlut_population {
     std::vector<float> init_state;   // initial SoA state (host copy)
     int items = kItems;              // neurons per thread of the update launch
 
-    int update_tiles() const { return (int)(stride / ((int64_t)kBlock * items)); }
+    // Neurons per update tile: the BDF kernels' is kBdfBlock (the granule's
+    // lists its spikes by as many).
+    int tile_size() const { return integ == EDLUT_BDF ? kBdfBlock : kBlock * items; }
+    int update_tiles() const { return (int)(stride / (int64_t)tile_size()); }
     bool granule_bdf() const { return model == EDLUT_GRANULE && integ == EDLUT_BDF; }
     // waves that give every neuron its kGrLanes lanes at once
     int granule_waves() const { return (int)(((int64_t)n * kGrLanes + kWave - 1) / kWave); }
@@ -349,7 +352,7 @@ struct edlut_population {
     // takes four neurons or more (200,000 cells: 495 us with 16, 543 us with
     // 8; 50,000: 175 and 178 us).
     int update_threads() const {
-        if (!granule_bdf()) return kBlock;
+        if (!granule_bdf()) return integ == EDLUT_BDF ? kBdfBlock : kBlock;
         const int w = (granule_waves() + n_cu - 1) / n_cu;
         return kWave * (w <= 4 ? 4 : (w < 32 ? 8 : 16));
     }
@@ -369,15 +372,12 @@ struct edlut_population {
         t.state = state;
         t.stride = stride;
         t.ndiff = nd;
-        t.cnt = cnt;
         t.fill = fill;
-        t.seg = seg;
         t.tile_flag = tile_flag;
-        t.bump = bump;
         t.par = par;
         t.b_ent = b_ent;
-        t.b_cap = b_cap;
-        t.err = err;
+        t.head = head;
+        t.node = node;
         return t;
     }
 
@@ -392,6 +392,38 @@ struct edlut_population {
         HIP_TRY(hipMalloc(&bdf_prev, np_rows * stride * elem));
         HIP_TRY(hipMemset(bdf_d, 0, nd_rows * stride * elem));
         HIP_TRY(hipMemset(bdf_prev, 0, np_rows * stride * elem));
+        return 0;
+    }
+
+    // Grow the queue of host-pushed events to hold `events` (the stream is idle
+    // between updates: an update ends with its spikes on the host).
+    int reserve_queue(int64_t events) {
+        if (events <= q_cap) return 0;
+        const int64_t cap = std::max<int64_t>(4096, events + events / 2);
+        if (cap > (1ll << 30)) return fail(EDLUT_E_CAP, "%lld input events queued for one update", (long long)events);
+        int32_t *t = nullptr;
+        FoldNode *nd = nullptr;
+        if (hipHostMalloc((void **)&t, (size_t)cap * 9, hipHostMallocDefault) != hipSuccess)
+            return fail(EDLUT_E_HIP, "hipHostMalloc failed");
+        const int rc = dalloc(&nd, (size_t)cap);
+        if (rc) {
+            (void)hipHostFree(t);
+            return rc;
+        }
+        float *w = (float *)(t + cap);
+        uint8_t *y = (uint8_t *)(w + cap);
+        if (q_n > 0) {
+            std::memcpy(t, q_tgt, sizeof(int32_t) * (size_t)q_n);
+            std::memcpy(w, q_w, sizeof(float) * (size_t)q_n);
+            std::memcpy(y, q_type, (size_t)q_n);
+        }
+        if (q_tgt) (void)hipHostFree(q_tgt);
+        if (node) (void)hipFree(node);
+        q_tgt = t;
+        q_w = w;
+        q_type = y;
+        node = nd;
+        q_cap = (int)cap;
         return 0;
     }
 
@@ -992,7 +1024,7 @@ int eq_resume(EqSim *S, int64_t first, int n_steps, double stop, hipStream_t st)
         E.dev.tile_count = E.net->tile_count;
         E.dev.staging = E.net->staging;
         E.dev.n_tiles = p->update_tiles();
-        E.dev.tile_size = kBlock * p->items;
+        E.dev.tile_size = p->tile_size();
     }
     std::vector<EqEmitter> dev, dev2;
     for (EqHostEm &E : S->em) dev.push_back(E.dev);
@@ -1041,9 +1073,9 @@ int model_param_count(int model) {
     return model >= 0 && model < 7 ? n[model] : -1;
 }
 
-// Neurons per thread of an ungrouped population's update kernel: the
-// granule's kernels hold two (19 state variables each; the BDF step keeps a
-// 15 x 15 matrix per neuron), every other kernel four.
+// Neurons per thread of an ungrouped population's update launch shape: two
+// for the granule (19 state variables each), four for every other kernel (the
+// BDF kernels hold one on each thread whatever the shape says).
 int plain_items(int model, int integrator) {
     (void)integrator;
     return model == EDLUT_GRANULE ? 2 : kItems;
@@ -1137,8 +1169,8 @@ struct MaskFreeTable {
             fn[6] = k_update_granule_bdf<false>;
             fn[7] = k_update_granule_bdf<true>;
         } else {
-            fn[6] = k_update_bdf<M, 15u, false, float, ITEMS>;
-            fn[7] = k_update_bdf<M, 15u, true, float, ITEMS>;
+            fn[6] = k_update_bdf<M, 15u, false, float>;
+            fn[7] = k_update_bdf<M, 15u, true, float>;
         }
         fn[8] = k_update<M, kBifEuler, 15u, false, ITEMS, false>;
         fn[9] = k_update<M, kBifEuler, 15u, true, ITEMS, false>;
@@ -1192,7 +1224,7 @@ UpdateFn pick_update(const edlut_population *p, bool ext) {
         return nullptr;
     }
     if (model == EDLUT_IZHIKEVICH || model == EDLUT_LIF_IS) {
-        if (p->items != kItems) return nullptr;
+        if (p->items != plain_items(model, integ)) return nullptr;
         static MaskFreeTable<IzhModel, kItems> iz;
         static MaskFreeTable<LifIsModel, kItems> li;
         return (model == EDLUT_IZHIKEVICH ? iz.fn : li.fn)[integ * 2 + (ext ? 1 : 0)];
@@ -1219,7 +1251,7 @@ UpdateFn pick_update(const edlut_population *p, bool ext) {
         const int idx = (integ * 4 + m) * 2 + (ext ? 1 : 0);
         return model == EDLUT_ADEX ? adex2.fn[idx] : lif2.fn[idx];
     }
-    if (p->items != kItems) return nullptr;
+    if (p->items != plain_items(model, integ)) return nullptr;
     if (integ >= EDLUT_BIFIXED_EULER) {
         static BifixedTable<AdExModel> adex_s;
         static BifixedTable<LIFModel> lif_s;
@@ -1251,10 +1283,8 @@ UpdateFn pick_update(const edlut_population *p, bool ext) {
     return nullptr;
 }
 
-int check_err(edlut_population *p) {
-    uint32_t e = 0;
-    HIP_TRY(hipMemcpyAsync(&e, p->err, sizeof(uint32_t), hipMemcpyDeviceToHost, p->stream));
-    HIP_TRY(hipStreamSynchronize(p->stream));
+// The error word's message and code.
+int err_code(uint32_t e) {
     if (e & 1u) return fail(EDLUT_E_STATE, "spike compaction look-back exceeded its spin limit");
     if (e & 2u)
         return fail(EDLUT_E_CAP, "spike log capacity exceeded (read and clear the log between runs, or raise "
@@ -1268,6 +1298,13 @@ int check_err(edlut_population *p) {
         return fail(EDLUT_E_ARG, "an input event in device memory names a target out of range or a synapse "
                                  "type that is not enabled (dropped)");
     return 0;
+}
+
+int check_err(edlut_population *p) {
+    uint32_t e = 0;
+    HIP_TRY(hipMemcpyAsync(&e, p->err, sizeof(uint32_t), hipMemcpyDeviceToHost, p->stream));
+    HIP_TRY(hipStreamSynchronize(p->stream));
+    return err_code(e);
 }
 
 UpdateArgs make_update_args(edlut_population *p, int32_t step) {
@@ -1325,6 +1362,9 @@ CompactArgs compact_args(int32_t *tile_count, int32_t *staging, int n_tiles, int
     c.log_cap = log_cap;
     c.err = err;
     c.step = step;
+    c.host_cnt = nullptr;
+    c.host_idx = nullptr;
+    c.host_cap = 0;
     c.clk_next = nullptr;
     c.clk_first = 0;
     c.clk_count = 0;
@@ -1343,18 +1383,12 @@ void launch_compact(hipStream_t st, int32_t *tile_count, int32_t *staging, int n
 }
 
 using RingFoldFn = void (*)(FoldTarget, RingEvents);
-template <int LANES>
-RingFoldFn ring_fold_fn(int pass) {
-    if (pass == kCount) return k_fold_ring<kCount, LANES>;
-    if (pass == kScatter) return k_fold_ring<kScatter, LANES>;
-    return k_fold_ring<kStatic, LANES>;
-}
-RingFoldFn pick_ring_fold(int pass, int lanes) {
+RingFoldFn pick_ring_fold(int lanes) {
     switch (lanes) {
-        case 8: return ring_fold_fn<8>(pass);
-        case 16: return ring_fold_fn<16>(pass);
-        case 32: return ring_fold_fn<32>(pass);
-        case 64: return ring_fold_fn<64>(pass);
+        case 8: return k_fold_ring<8>;
+        case 16: return k_fold_ring<16>;
+        case 32: return k_fold_ring<32>;
+        case 64: return k_fold_ring<64>;
         default: return nullptr;
     }
 }
@@ -1387,22 +1421,17 @@ CompactFoldFn pick_compact_fold(int lanes) {
 
 // The network-mode fold (one pass into the keys' fixed segments).
 int launch_ring_fold(const FoldTarget &t, hipStream_t st, const RingEvents &re, int lanes, int blocks) {
-    RingFoldFn f = pick_ring_fold(kStatic, lanes);
+    RingFoldFn f = pick_ring_fold(lanes);
     if (!f) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
     hipLaunchKernelGGL(f, dim3(blocks), dim3(kBlock), 0, st, t, re);
     return 0;
 }
 
-// Both passes of the fold of host-pushed events (plug-in mode).
-int launch_push_fold(edlut_population *p, int par, int n_events, const PushEvents *pe) {
-    if (n_events == 0) return 0;
-    FoldTarget t = p->fold_target(par, false);
-    int nb = (n_events + kBlock - 1) / kBlock;
-    if (nb > 4096) nb = 4096;
-    hipLaunchKernelGGL((k_fold_push<kCount>), dim3(nb), dim3(kBlock), 0, p->stream, t, *pe);
-    hipLaunchKernelGGL((k_fold_push<kScatter>), dim3(nb), dim3(kBlock), 0, p->stream, t, *pe);
-    HIP_TRY(hipGetLastError());
-    return 0;
+// The fold of host-pushed events (plug-in mode).
+void launch_push_fold(const FoldTarget &t, const PushEvents &pe, hipStream_t st) {
+    if (pe.n == 0) return;
+    const int nb = std::min((pe.n + kBlock - 1) / kBlock, 4096);
+    hipLaunchKernelGGL(k_fold_push, dim3(nb), dim3(kBlock), 0, st, t, pe);
 }
 
 __global__ void k_fill_i32(int32_t *p, int64_t n, int32_t v) {
@@ -1756,12 +1785,9 @@ int create_population(int model, int integrator, int bdf_order, const float *par
     if ((rc = dalloc(&p->spk_idx, n_neurons))) return cleanup(rc);
     if ((rc = dalloc(&p->spk_cnt, 1))) return cleanup(rc);
     if ((rc = dalloc(&p->err, 1))) return cleanup(rc);
-    if ((rc = dalloc(&p->cnt, (size_t)3 * p->stride))) return cleanup(rc);
+    if ((rc = dalloc(&p->head, (size_t)3 * p->stride))) return cleanup(rc);
     if ((rc = dalloc(&p->fill, (size_t)3 * p->stride))) return cleanup(rc);
-    if ((rc = dalloc(&p->seg, (size_t)3 * p->stride))) return cleanup(rc);
     if ((rc = dalloc(&p->tile_flag, max_tiles))) return cleanup(rc);
-    if ((rc = dalloc(&p->bump, 2))) return cleanup(rc);
-    if ((rc = p->reserve_events(1u << 16))) return cleanup(rc);
     if (model == EDLUT_LIF || model == EDLUT_PURKINJE || model == EDLUT_LIF_IS) {
         if ((rc = dalloc(&p->last_spike, p->stride))) return cleanup(rc);
         std::vector<int32_t> never(p->stride, -(1 << 30));
@@ -1771,7 +1797,7 @@ int create_population(int model, int integrator, int bdf_order, const float *par
     }
     if (hipHostMalloc((void **)&p->h_spk, sizeof(int32_t) * n_neurons, hipHostMallocDefault) !=
             hipSuccess ||
-        hipHostMalloc((void **)&p->h_cnt, sizeof(int32_t), hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc((void **)&p->h_cnt, 2 * sizeof(int32_t), hipHostMallocDefault) != hipSuccess)
         return cleanup(fail(EDLUT_E_HIP, "hipHostMalloc failed"));
 
     // initial state (VectorNeuronState_GPU_C_INTERFACE.cu:66-131), per group
@@ -1791,11 +1817,9 @@ int create_population(int model, int integrator, int bdf_order, const float *par
               hipMemset(p->tile_count, 0, sizeof(int32_t) * padded_tiles((int)max_tiles)) == hipSuccess &&
               hipMemset(p->spk_cnt, 0, sizeof(int32_t)) == hipSuccess &&
               hipMemset(p->err, 0, sizeof(uint32_t)) == hipSuccess &&
-              hipMemset(p->cnt, 0, sizeof(uint32_t) * 3 * p->stride) == hipSuccess &&
+              hipMemset(p->head, 0, sizeof(uint32_t) * 3 * p->stride) == hipSuccess &&
               hipMemset(p->fill, 0, sizeof(uint32_t) * 3 * p->stride) == hipSuccess &&
-              hipMemset(p->tile_flag, 0, sizeof(uint32_t) * max_tiles) == hipSuccess &&
-              hipMemset(p->seg, 0xff, sizeof(uint64_t) * 3 * p->stride) == hipSuccess &&
-              hipMemset(p->bump, 0, 2 * sizeof(uint64_t)) == hipSuccess;
+              hipMemset(p->tile_flag, 0, sizeof(uint32_t) * max_tiles) == hipSuccess;
     if (!ok) return cleanup(fail(EDLUT_E_HIP, "device initialisation failed"));
     *out = p;
     return 0;
@@ -1844,13 +1868,13 @@ int edlut_population_destroy(edlut_population *p) {
     void *dev[] = {p->chan, p->bdf_c, p->bdf_d, p->bdf_prev, p->bdf_st, p->bdf_ws, p->bdf_ws_count,
                    p->bdf_bits, p->bdf_done,
                    p->state, p->last_spike, p->exp_lut, p->nmda_lut, p->refr, p->tile_count,
-                   p->staging, p->spk_idx, p->spk_cnt, p->err, p->cnt, p->fill, p->seg,
-                   p->tile_flag, p->bump, p->b_ent, p->e_tgt,
-                   p->e_type, p->e_w, p->d_groups, p->d_chunk_group};
+                   p->staging, p->spk_idx, p->spk_cnt, p->err, p->head, p->node, p->fill,
+                   p->tile_flag, p->b_ent, p->d_groups, p->d_chunk_group};
     for (void *q : dev)
         if (q) (void)hipFree(q);
     if (p->h_spk) (void)hipHostFree(p->h_spk);
     if (p->h_cnt) (void)hipHostFree(p->h_cnt);
+    if (p->q_tgt) (void)hipHostFree(p->q_tgt);
     if (p->stream) (void)hipStreamDestroy(p->stream);
     delete p;
     return 0;
@@ -1883,9 +1907,14 @@ int edlut_population_push_inputs(edlut_population *p, const int32_t *target, con
         if (!(p->mask & (1u << type[i])))
             return fail(EDLUT_E_ARG, "event %d: synapse type %d is not enabled", i, type[i]);
     }
-    p->q_tgt.insert(p->q_tgt.end(), target, target + n);
-    p->q_type.insert(p->q_type.end(), type, type + n);
-    p->q_w.insert(p->q_w.end(), weight, weight + n);
+    if (n == 0) return 0;
+    HIP_TRY(hipSetDevice(p->device));
+    const int rc = p->reserve_queue((int64_t)p->q_n + n);
+    if (rc) return rc;
+    std::memcpy(p->q_tgt + p->q_n, target, sizeof(int32_t) * (size_t)n);
+    std::memcpy(p->q_w + p->q_n, weight, sizeof(float) * (size_t)n);
+    std::memcpy(p->q_type + p->q_n, type, (size_t)n);
+    p->q_n += n;
     return 0;
 }
 
@@ -1899,61 +1928,43 @@ int edlut_population_set_ext_current(edlut_population *p, const float *current) 
     return 0;
 }
 
+// Spikes of an update that the compaction writes to host memory itself; more
+// are copied back as a whole.
+static constexpr int kHostSpikes = 4096;
+
 int edlut_population_update(edlut_population *p, int64_t step, int *n_spikes) {
     if (!p) return fail(EDLUT_E_ARG, "population is null");
     if (step < 1 || step > (1ll << 30)) return fail(EDLUT_E_ARG, "update index out of range");
     HIP_TRY(hipSetDevice(p->device));
+    UpdateFn fn = pick_update(p, false);
+    if (!fn) return fail(EDLUT_E_ARG, "no update kernel for this model, integrator and synapse set");
     // 1. ordered fold of the queued input spikes
-    const int ne = (int)p->q_tgt.size();
-    const int par = (int)(++p->upd_seq & 1u);
-    int rc0 = 0;
-    if (ne > 0) {
-        if (ne > p->e_cap) {
-            (void)hipFree(p->e_tgt);
-            (void)hipFree(p->e_type);
-            (void)hipFree(p->e_w);
-            p->e_tgt = nullptr;
-            p->e_type = nullptr;
-            p->e_w = nullptr;
-            int rc;
-            int cap = ne < 4096 ? 4096 : ne * 2;
-            if ((rc = dalloc(&p->e_tgt, cap)) || (rc = dalloc(&p->e_type, cap)) ||
-                (rc = dalloc(&p->e_w, cap)))
-                return rc;
-            p->e_cap = cap;
-        }
-        HIP_TRY(hipMemcpyAsync(p->e_tgt, p->q_tgt.data(), sizeof(int32_t) * ne, hipMemcpyHostToDevice, p->stream));
-        HIP_TRY(hipMemcpyAsync(p->e_type, p->q_type.data(), ne, hipMemcpyHostToDevice, p->stream));
-        HIP_TRY(hipMemcpyAsync(p->e_w, p->q_w.data(), sizeof(float) * ne, hipMemcpyHostToDevice, p->stream));
-        if ((rc0 = p->reserve_events((uint64_t)ne))) return rc0;
-        PushEvents pe{p->e_tgt, p->e_type, p->e_w, ne, (int32_t)p->n, p->mask & 7u, p->err};
-        int rc = launch_push_fold(p, par, ne, &pe);
-        if (rc) return rc;
-    }
+    const FoldTarget t = p->fold_target((int)(++p->upd_seq & 1u));
+    launch_push_fold(t, PushEvents{p->q_tgt, p->q_type, p->q_w, p->q_n, (int32_t)p->n, p->mask & 7u, p->err}, p->stream);
     // 2. integrate, detect, compact
     UpdateArgs a = make_update_args(p, (int32_t)step);
     a.out = TileOut{p->tile_count, p->staging};
-    a.fold = p->fold_target(par);
-    UpdateFn fn = pick_update(p, false);
-    if (!fn) return fail(EDLUT_E_ARG, "no update kernel for this model, integrator and synapse set");
+    a.fold = t;
     p->started = true;
     const int tiles = p->update_tiles();
     hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), p->stream, a);
-    launch_compact(p->stream, p->tile_count, p->staging, tiles, kBlock * p->items, p->spk_idx, p->spk_cnt,
-                   1, 0, nullptr, nullptr, nullptr, 0, p->err, StepRef{nullptr, (int32_t)step});
+    CompactArgs c = compact_args(p->tile_count, p->staging, tiles, p->tile_size(), p->spk_idx, p->spk_cnt, 1, 0,
+                                 nullptr, nullptr, nullptr, 0, p->err, StepRef{nullptr, (int32_t)step});
+    c.host_cnt = p->h_cnt;
+    c.host_idx = p->h_spk;
+    c.host_cap = kHostSpikes;
+    hipLaunchKernelGGL(k_compact, dim3(compact_blocks(tiles)), dim3(kBlock), 0, p->stream, c);
     HIP_TRY(hipGetLastError());
-    // 3. hand the compacted spikes back (synchronous, like the reference)
-    HIP_TRY(hipMemcpyAsync(p->h_cnt, p->spk_cnt, sizeof(int32_t), hipMemcpyDeviceToHost, p->stream));
+    // 3. hand the compacted spikes back (synchronous, like the reference): the
+    // compaction wrote them to host memory, up to kHostSpikes of them
     HIP_TRY(hipStreamSynchronize(p->stream));
-    const int ns = *p->h_cnt;
-    if (ns > 0) {
+    const int ns = p->h_cnt[0];
+    if (ns > kHostSpikes) {
         HIP_TRY(hipMemcpyAsync(p->h_spk, p->spk_idx, sizeof(int32_t) * ns, hipMemcpyDeviceToHost, p->stream));
         HIP_TRY(hipStreamSynchronize(p->stream));
     }
-    p->q_tgt.clear();
-    p->q_type.clear();
-    p->q_w.clear();
-    int rc = check_err(p);
+    p->q_n = 0;
+    const int rc = err_code((uint32_t)p->h_cnt[1]);
     if (rc) return rc;
     p->last_n_spikes = ns;
     if (n_spikes) *n_spikes = ns;
@@ -1965,12 +1976,11 @@ int edlut_population_update(edlut_population *p, int64_t step, int *n_spikes) {
 namespace {
 
 // ---------------------------------------------------------------------------
-// Allocation-free update: the input fold's event buffer (order keys and
-// weights of the step's events, grouped by target) lives in this file-scope
-// device array instead of the population's growable buffer.  Each device
+// Allocation-free update: the list nodes of the input fold's events live in
+// this file-scope device array instead of the population's growable one.  Each device
 // holds its own copy at its own address, looked up once per device.
 constexpr int64_t kNoAllocMaxEvents = 1 << 20;
-static __device__ __align__(256) uint8_t scratch[kNoAllocMaxEvents * sizeof(FoldEntry)];
+static __device__ __align__(256) uint8_t scratch[kNoAllocMaxEvents * sizeof(FoldNode)];
 
 constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu;
@@ -2005,7 +2015,7 @@ int edlut_population_update_noalloc(edlut_population *p, int64_t step, const int
         return fail(EDLUT_E_CAP, "%d input events exceed the allocation-free update's maximum of %lld", n_events,
                     (long long)kNoAllocMaxEvents);
     if (!spk_idx || !spk_cnt) return fail(EDLUT_E_ARG, "null spike output");
-    if (!p->q_tgt.empty())
+    if (p->q_n > 0)
         return fail(EDLUT_E_STATE, "input events queued by edlut_population_push_inputs: use edlut_population_update");
     UpdateFn fn = pick_update(p, false);
     if (!fn) return fail(EDLUT_E_ARG, "no update kernel for this model, integrator and synapse set");
@@ -2015,17 +2025,9 @@ int edlut_population_update_noalloc(edlut_population *p, int64_t step, const int
     if (rc) return rc;
     const hipStream_t st = stream ? (hipStream_t)stream : p->stream;
     // 1. ordered fold of the events (position in the arrays = delivery order)
-    const int par = (int)(++p->upd_seq & 1u);
-    FoldTarget t = p->fold_target(par);
-    t.b_ent = (FoldEntry *)base;
-    t.b_cap = (uint64_t)kNoAllocMaxEvents;
-    if (n_events > 0) {
-        const PushEvents pe{target, type, weight, n_events, (int32_t)p->n, p->mask & 7u, p->err};
-        int nb = (n_events + kBlock - 1) / kBlock;
-        if (nb > 4096) nb = 4096;
-        hipLaunchKernelGGL((k_fold_push<kCount>), dim3(nb), dim3(kBlock), 0, st, t, pe);
-        hipLaunchKernelGGL((k_fold_push<kScatter>), dim3(nb), dim3(kBlock), 0, st, t, pe);
-    }
+    FoldTarget t = p->fold_target((int)(++p->upd_seq & 1u));
+    t.node = (FoldNode *)base;
+    launch_push_fold(t, PushEvents{target, type, weight, n_events, (int32_t)p->n, p->mask & 7u, p->err}, st);
     // 2. integrate, detect, compact into the caller's spike list
     UpdateArgs a = make_update_args(p, (int32_t)step);
     a.out = TileOut{p->tile_count, p->staging};
@@ -2033,7 +2035,7 @@ int edlut_population_update_noalloc(edlut_population *p, int64_t step, const int
     p->started = true;
     const int tiles = p->update_tiles();
     hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), st, a);
-    launch_compact(st, p->tile_count, p->staging, tiles, kBlock * p->items, spk_idx, spk_cnt, 1, 0, nullptr,
+    launch_compact(st, p->tile_count, p->staging, tiles, p->tile_size(), spk_idx, spk_cnt, 1, 0, nullptr,
                    nullptr, nullptr, 0, p->err, StepRef{nullptr, (int32_t)step});
     HIP_TRY(hipGetLastError());
     return 0;
@@ -2564,7 +2566,7 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
         a.clk_count = (int32_t)n->clk_count;
     }
     hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), p->stream, a);
-    CompactArgs c = compact_args(n->tile_count, n->staging, tiles, kBlock * p->items, n->own_ring_idx,
+    CompactArgs c = compact_args(n->tile_count, n->staging, tiles, p->tile_size(), n->own_ring_idx,
                                  n->own_ring_cnt, n->ring, p->n, n->log_cap ? n->log_step : nullptr,
                                  n->log_cap ? n->log_idx : nullptr, n->log_count, n->log_cap, p->err, step);
     if (n->clk) {
@@ -2739,7 +2741,7 @@ static int build_segments(edlut_network *n) {
 // the timing window set.  Returns the update kernel through *fn.
 static int run_prepare(edlut_network *n, int64_t first_step, int n_steps, UpdateFn *fn) {
     edlut_population *p = n->pop;
-    if (!p->q_tgt.empty()) return fail(EDLUT_E_STATE, "queued host inputs are not used in network mode");
+    if (p->q_n > 0) return fail(EDLUT_E_STATE, "queued host inputs are not used in network mode");
     if (n->fold_ready >= 0 && (first_step != n->fold_ready || n->seg_dirty)) {
         // events folded ahead for an update that will not run next (or into
         // segments about to change): drop them, the fold is redone
@@ -2768,7 +2770,6 @@ static int run_prepare(edlut_network *n, int64_t first_step, int n_steps, Update
             HIP_TRY(hipMemcpy(s.log_count, sc, sizeof(sc), hipMemcpyHostToDevice));
         }
     }
-    HIP_TRY(hipMemsetAsync(p->bump, 0, 2 * sizeof(uint64_t), p->stream));
     if (n->plastic) {
         // update time of the step before the run, in its ring slot
         const double t0 = n->time_of(first_step - 1);
@@ -3507,9 +3508,8 @@ int edlut_network_reset(edlut_network *n) {
         HIP_TRY(hipMemsetAsync(s.syn.post, 0, sizeof(float) * s.nsyn, p->stream));
         HIP_TRY(hipMemsetAsync(s.syn.last, 0, sizeof(double) * s.nsyn, p->stream));
     }
-    HIP_TRY(hipMemsetAsync(p->cnt, 0, sizeof(uint32_t) * 3 * p->stride, p->stream));
+    HIP_TRY(hipMemsetAsync(p->head, 0, sizeof(uint32_t) * 3 * p->stride, p->stream));
     HIP_TRY(hipMemsetAsync(p->fill, 0, sizeof(uint32_t) * 3 * p->stride, p->stream));
-    HIP_TRY(hipMemsetAsync(p->seg, 0xff, sizeof(uint64_t) * 3 * p->stride, p->stream));
     HIP_TRY(hipMemsetAsync(p->tile_flag, 0, sizeof(uint32_t) * (p->stride / kFlagTile), p->stream));
     n->fold_ready = -1;
     HIP_TRY(hipStreamSynchronize(p->stream));
@@ -3524,7 +3524,7 @@ int edlut_network_set_launch(edlut_network *n, int items, int fold_lanes, int fo
     const bool two_or_four = p->grouped || plain_two_items(p);
     if (two_or_four ? (items != 2 && items != 4) : items != fixed)
         return fail(EDLUT_E_ARG, "items per thread must be %s", two_or_four ? "2 or 4" : (fixed == 2 ? "2" : "4"));
-    if (!pick_ring_fold(kCount, fold_lanes)) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
+    if (!pick_ring_fold(fold_lanes)) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
     if (fold_blocks < 1 || fold_blocks > 65536) return fail(EDLUT_E_ARG, "fold blocks must be in [1, 65536]");
     p->items = items;
     n->fold_lanes = fold_lanes;

@@ -419,15 +419,13 @@ struct GranuleGroup {
 constexpr int kGrBdfThreads = 1024;   // largest workgroup: four waves per SIMD (128 registers each)
 template <bool EXT>
 __global__ __launch_bounds__(kGrBdfThreads) void k_update_granule_bdf(UpdateArgs a) {
-    constexpr int TILE = kFlagTile, L = kGrLanes;
+    constexpr int TILE = kBdfBlock, L = kGrLanes;   // spike lists by kBdfBlock neurons
+    static_assert(TILE == kFlagTile, "one fold flag per spike list");
     const int32_t step = a.step.get();
     clock_begin(a, step);
     const int par = a.fold.par_by_step ? (step & 1) : a.fold.par;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        a.fold.bump[par ^ 1] = 0ull;
-        // the next step hands out working-storage slots from the other parity
-        if (a.bdf.ws_count) a.bdf.ws_count[par ^ 1] = 0u;
-    }
+    // the next step hands out working-storage slots from the other parity
+    if (blockIdx.x == 0 && threadIdx.x == 0 && a.bdf.ws_count) a.bdf.ws_count[par ^ 1] = 0u;
     const uint32_t step_key = EXT ? drive_step_key(a.ext.seed, step) : 0u;
     __shared__ float s_bdfc[49];
     extern __shared__ float4 s_chan[];

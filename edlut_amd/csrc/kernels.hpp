@@ -23,17 +23,16 @@ constexpr int kBifixed = 3;
 //
 // Every input event of a step is (key = type*stride + target, order, w); the
 // CPU reference adds them one by one into the state, in `order`.  The fold
-// reproduces that sequence exactly, for any event density, in two passes
-// plus a tail in the update kernel:
+// reproduces that sequence exactly, for any event density, in one pass over
+// the events and a tail in the update kernel:
 //
-//   count    per-key event counts (atomic increments)
-//   scatter  keys with one event add it directly -- no ordering question;
-//            for the others the first arrival reserves a contiguous segment
-//            of the event buffer, every event drops (order, w) into it, and
-//            the target's tile is flagged
-//   update   in flagged tiles each neuron sorts its keys' segments by order
-//            and folds them sequentially before integrating, then clears the
-//            key's counters
+//   events   network mode: each event takes the next free entry of its key's
+//            fixed segment of the event buffer; plug-in mode (any number of
+//            events per key): event q becomes node q of its key's list.  The
+//            target's tile is flagged.
+//   update   in flagged tiles each neuron brings its keys' events into order
+//            and adds them to the conductance one by one before integrating,
+//            then clears the key
 //
 // The event buffer can hold every event of a step (one per synapse) in the
 // network mode, so it cannot overflow there.
@@ -41,9 +40,8 @@ constexpr int kBifixed = 3;
 constexpr int kItems = 4;                    // neurons per thread in the update kernels
 constexpr int kUpdTile = kBlock * kItems;    // neurons per update tile (kItems per thread)
 constexpr int kFlagTile = 512;               // neurons per fold flag (smallest update tile)
+constexpr int kBdfBlock = 512;               // threads, and neurons, of a BDF update tile
 constexpr int kGroupAlign = 256;             // grouped populations: groups start on this
-constexpr uint64_t kSegEmpty = ~0ull;
-constexpr uint64_t kSegBusy = ~0ull - 1ull;
 
 // One queued event of the fold: its order key and weight in one 16-byte
 // entry, so that scattering an event writes one line.
@@ -53,20 +51,24 @@ struct FoldEntry {
     uint32_t pad;
 };
 
+// One host-pushed event: its weight and the event that reached the key's list
+// before it (1 + its number; 0 ends the list).
+struct FoldNode {
+    uint32_t next;
+    float w;
+};
+
 struct FoldTarget {
     float *state;
     int64_t stride;
     int ndiff;
-    uint32_t *cnt;       // per key: events this step
-    uint32_t *fill;      // per key: events scattered so far
-    uint64_t *seg;       // per key: segment start (kSegEmpty when none)
-    uint32_t *tile_flag; // per kFlagTile neurons: some key there has >= 2 events
-    uint64_t *bump;      // [2] event-buffer allocator, by step parity
+    uint32_t *fill;      // network mode, per key: events this step
+    uint32_t *tile_flag; // per kFlagTile neurons: some key there has an event
     int par;             // parity of this step, unless par_by_step
     int par_by_step;     // parity = update index & 1 (network mode)
-    FoldEntry *b_ent;    // event buffer (order key, weight)
-    uint64_t b_cap;
-    uint32_t *err;       // bit 2: event buffer overflow, bit 3: spin limit
+    FoldEntry *b_ent;    // network mode: event buffer (order key, weight)
+    uint32_t *head;      // plug-in mode, per key: 1 + its last listed event (0: none)
+    FoldNode *node;      // plug-in mode: the step's events
     // network mode: fixed segment of each key (prefix of the keys' synapse
     // counts; a synapse carries at most one event per step), null otherwise
     const uint64_t *seg_off;
@@ -101,55 +103,12 @@ __device__ __forceinline__ float *g_ptr(const FoldTarget &t, uint64_t key) {
     return t.state + (int64_t)(t.ndiff + (int)type) * t.stride + (int64_t)tgt;
 }
 
-enum FoldPass { kCount = 0, kScatter = 1, kStatic = 2 };
-
-template <int PASS>
-__device__ __forceinline__ void fold_event(const FoldTarget &t, int par, uint64_t key, uint64_t ord,
-                                           float w) {
-    if (PASS == kStatic) {
-        // network mode, one pass: the key's fixed segment, next free entry
-        const uint32_t pos = atomicAdd(&t.fill[key], 1u);
-        const uint64_t at = t.seg_off[key] + pos;
-        t.b_ent[at] = FoldEntry{ord, w, 0u};
-        if (pos == 0u) t.tile_flag[(key % (uint64_t)t.stride) / kFlagTile] = 1u;
-        return;
-    }
-    if (PASS == kCount) {
-        atomicAdd(&t.cnt[key], 1u);
-        return;
-    }
-    const uint32_t c = t.cnt[key];
-    if (c == 1u) {
-        float *g = g_ptr(t, key);
-        *g = *g + w;
-        t.cnt[key] = 0u;
-        return;
-    }
-    // Reserve the key's segment (first arrival) -- every lane does this step
-    // before any lane waits, so a wave never waits on one of its own lanes.
-    const uint64_t prev = atomicCAS((unsigned long long *)&t.seg[key], kSegEmpty, kSegBusy);
-    if (prev == kSegEmpty) {
-        const uint64_t base = atomicAdd((unsigned long long *)&t.bump[par], (unsigned long long)c);
-        __hip_atomic_store(&t.seg[key], base, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const uint64_t tgt = key % (uint64_t)t.stride;
-        t.tile_flag[tgt / kFlagTile] = 1u;
-    }
-    uint64_t base = __hip_atomic_load(&t.seg[key], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t spins = 0;
-    while (base == kSegBusy) {
-        if (++spins > (1u << 22)) {
-            atomicOr(t.err, 8u);
-            return;
-        }
-        __builtin_amdgcn_s_sleep(1);
-        base = __hip_atomic_load(&t.seg[key], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    const uint64_t pos = base + atomicAdd(&t.fill[key], 1u);
-    if (pos < t.b_cap) {
-        t.b_ent[pos] = FoldEntry{ord, w, 0u};
-    } else {
-        atomicOr(t.err, 4u);
-    }
+// Network mode: the key's fixed segment, next free entry.
+__device__ __forceinline__ void fold_event(const FoldTarget &t, uint64_t key, uint64_t ord, float w) {
+    const uint32_t pos = atomicAdd(&t.fill[key], 1u);
+    const uint64_t at = t.seg_off[key] + pos;
+    t.b_ent[at] = FoldEntry{ord, w, 0u};
+    if (pos == 0u) t.tile_flag[(key % (uint64_t)t.stride) / kFlagTile] = 1u;
 }
 
 // Network mode: folds the m >= 1 events of `key` (its fixed segment) into g
@@ -188,32 +147,40 @@ __device__ __attribute__((noinline)) float fold_static(uint32_t *fill, const uin
     return g;
 }
 
-// Folds the segment of `key` (m >= 2 events) into g in order and clears the
-// key's counters.  Called by the update kernel for its own neuron, out of
-// line so the common path keeps its small register budget; the segment is
-// sorted in place in the event buffer (insertion sort: segments are short).
-__device__ __attribute__((noinline)) float fold_segment(uint32_t *cnt, uint32_t *fill,
-                                                        uint64_t *seg, FoldEntry *e, uint64_t b_cap,
-                                                        uint32_t *err, uint64_t key,
-                                                        uint32_t m, float g) {
-    const uint64_t b = seg[key];
-    if (b == kSegEmpty || b == kSegBusy || b + m > b_cap) {
-        atomicOr(err, 4u);
+// Plug-in mode: adds the events listed from `hd` to g in the order of their
+// numbers and clears the list.  Each walk finds the next four of them, so a
+// list of up to four takes two walks.
+__device__ __attribute__((noinline)) float fold_list(uint32_t *head, const FoldNode *node, uint64_t key, uint32_t hd,
+                                                     float g) {
+    uint32_t last = 0u;
+    const FoldNode first = node[hd - 1u];
+    if (first.next == 0u) {
+        g = g + first.w;
     } else {
-        for (uint32_t j = 1; j < m; j++) {
-            const FoldEntry k = e[b + j];
-            int64_t i = (int64_t)j - 1;
-            while (i >= 0 && e[b + i].ord > k.ord) {
-                e[b + i + 1] = e[b + i];
-                --i;
+        for (;;) {
+            uint32_t b0 = ~0u, b1 = ~0u, b2 = ~0u, b3 = ~0u;
+            float w0 = 0.0f, w1 = 0.0f, w2 = 0.0f, w3 = 0.0f;
+            for (uint32_t q = hd; q != 0u;) {
+                const FoldNode e = node[q - 1u];
+                if (q > last && q < b3) {
+                    b3 = q;
+                    w3 = e.w;
+                    if (b3 < b2) { const uint32_t t = b2; b2 = b3; b3 = t; const float u = w2; w2 = w3; w3 = u; }
+                    if (b2 < b1) { const uint32_t t = b1; b1 = b2; b2 = t; const float u = w1; w1 = w2; w2 = u; }
+                    if (b1 < b0) { const uint32_t t = b0; b0 = b1; b1 = t; const float u = w0; w0 = w1; w1 = u; }
+                }
+                q = e.next;
             }
-            e[b + i + 1] = k;
+            if (b0 == ~0u) break;
+            g = g + w0;
+            if (b1 != ~0u) g = g + w1;
+            if (b2 != ~0u) g = g + w2;
+            if (b3 == ~0u) break;
+            g = g + w3;
+            last = b3;
         }
-        for (uint32_t j = 0; j < m; j++) g = g + e[b + j].w;
     }
-    cnt[key] = 0u;
-    fill[key] = 0u;
-    seg[key] = kSegEmpty;
+    head[key] = 0u;
     return g;
 }
 
@@ -299,6 +266,18 @@ __device__ __forceinline__ void clear_tile_flag(uint32_t *flags, int tile) {
     for (int q = 0; q < F; q++) flags[tile * F + q] = 0u;
 }
 
+// The queued events of neuron i's key of synapse type ty, added to its
+// conductance g in order.
+__device__ __forceinline__ float fold_key(const UpdateArgs &a, int32_t step, int ty, uint32_t i, float g) {
+    const uint64_t key = (uint64_t)ty * (uint64_t)a.stride + (uint64_t)i;
+    if (a.fold.seg_off) {
+        const uint32_t m = a.fold.fill[key];
+        return m >= 1u ? fold_static(a.fold.fill, a.fold.seg_off, a.fold.b_ent, a.fold.rtab, step & 1, key, m, g) : g;
+    }
+    const uint32_t hd = a.fold.head[key];
+    return hd ? fold_list(a.fold.head, a.fold.node, key, hd, g) : g;
+}
+
 // One tile = kBlock*ITEMS neurons in the wave-major layout of tile_neuron:
 // each lane handles ITEMS neurons kWave apart (each item is one coalesced row
 // access per wave).  All loads are issued first, the ITEMS neurons are
@@ -313,7 +292,6 @@ __global__ __launch_bounds__(kBlock) void k_update(UpdateArgs a) {
     const int tile = blockIdx.x;
     const int32_t step = a.step.get();
     clock_begin(a, step);
-    const int par = a.fold.par_by_step ? (step & 1) : a.fold.par;
     __shared__ uint32_t s_flag;
     // the tile's fold flag is read alongside the state loads (the barrier
     // that publishes it comes after them)
@@ -336,7 +314,6 @@ __global__ __launch_bounds__(kBlock) void k_update(UpdateArgs a) {
     float *__restrict__ row[M::NV];
 #pragma unroll
     for (int j = 0; j < M::NV; j++) row[j] = a.state + (int64_t)j * a.stride;
-    const int64_t ld = a.stride;
     const uint32_t step_key = EXT ? drive_step_key(dseed, step) : 0u;
     int idx[ITEMS];
     bool live[ITEMS];
@@ -364,31 +341,17 @@ __global__ __launch_bounds__(kBlock) void k_update(UpdateArgs a) {
     if (threadIdx.x == 0) {
         s_flag = flag;
         if (flag) clear_tile_flag<T>(a.fold.tile_flag, tile);
-        // the next step's fold allocates from the other parity: clear it
-        if (tile == 0) a.fold.bump[par ^ 1] = 0ull;
     }
     __syncthreads();
     if (s_flag) {
-        // events of keys with several inputs this step, in delivery order
+        // the step's input events, in delivery order
 #pragma unroll
         for (int n = 0; n < ITEMS; n++) {
             if (!live[n]) continue;
 #pragma unroll
             for (int ty = 0; ty < 3; ty++) {
                 if (!(MASK & (1u << ty))) continue;
-                const uint64_t key = (uint64_t)ty * (uint64_t)ld + (uint64_t)idx[n];
-                if (a.fold.seg_off) {
-                    const uint32_t m = a.fold.fill[key];
-                    if (m >= 1u)
-                        s[n][M::EXC + ty] = fold_static(a.fold.fill, a.fold.seg_off, a.fold.b_ent,
-                                                        a.fold.rtab, step & 1, key, m, s[n][M::EXC + ty]);
-                    continue;
-                }
-                const uint32_t m = a.fold.cnt[key];
-                if (m >= 2u)
-                    s[n][M::EXC + ty] = fold_segment(a.fold.cnt, a.fold.fill, a.fold.seg, a.fold.b_ent,
-                                                     a.fold.b_cap, a.fold.err, key, m,
-                                                     s[n][M::EXC + ty]);
+                s[n][M::EXC + ty] = fold_key(a, step, ty, (uint32_t)idx[n], s[n][M::EXC + ty]);
             }
         }
     }
@@ -485,19 +448,6 @@ __global__ __launch_bounds__(kBlock) void k_update(UpdateArgs a) {
 }
 
 
-// The queued events of neuron i's key of synapse type ty, added to its
-// conductance g in order.
-__device__ __forceinline__ float fold_key(const UpdateArgs &a, int32_t step, int ty, uint32_t i, float g) {
-    const uint64_t key = (uint64_t)ty * (uint64_t)a.stride + (uint64_t)i;
-    if (a.fold.seg_off) {
-        const uint32_t m = a.fold.fill[key];
-        return m >= 1u ? fold_static(a.fold.fill, a.fold.seg_off, a.fold.b_ent, a.fold.rtab, step & 1, key, m, g) : g;
-    }
-    const uint32_t m = a.fold.cnt[key];
-    return m >= 2u ? fold_segment(a.fold.cnt, a.fold.fill, a.fold.seg, a.fold.b_ent, a.fold.b_cap, a.fold.err, key,
-                                  m, g) : g;
-}
-
 // Loads the state of neuron i at the start of a BDF step into sf: the row
 // values, the ordered fold of its multi-event keys when its tile's fold flag
 // is set, and the external drive.
@@ -540,24 +490,23 @@ __device__ __forceinline__ void bdf_store(const UpdateArgs &a, float *__restrict
     }
 }
 
-// BDF update: one neuron at a time per thread (data-dependent Newton
-// iterations), ITEMS neurons per thread in the item-major layout of
-// tile_spikes_item_major (a small population takes one neuron per thread).
-// T = double runs the whole BDF step in double (FP64 Newton mode); the state
-// is stored back in float.
-template <class M, unsigned MASK, bool EXT, typename T, int ITEMS = kItems>
-__global__ __launch_bounds__(kBlock) void k_update_bdf(UpdateArgs a) {
-    constexpr int TILE = kBlock * ITEMS;
+// BDF update: one neuron per thread (the Newton iteration is a serial chain of
+// data-dependent length, so a second neuron on the thread doubles the kernel
+// wherever the population leaves SIMDs idle).  T = double runs the whole BDF
+// step in double (FP64 Newton mode); the state is stored back in float.
+// 4,099 HH cells, FP64 Newton: 41 us per launch; with four neurons on each of 256
+// threads 109 us.
+template <class M, unsigned MASK, bool EXT, typename T>
+__global__ __launch_bounds__(kBdfBlock) void k_update_bdf(UpdateArgs a) {
+    constexpr int TILE = kBdfBlock;
     static_assert(TILE % kFlagTile == 0, "update tiles cover whole fold flags");
     const int tile = blockIdx.x;
     const int32_t step = a.step.get();
     clock_begin(a, step);
-    const int par = a.fold.par_by_step ? (step & 1) : a.fold.par;
     __shared__ uint32_t s_flag;
     if (threadIdx.x == 0) {
         s_flag = take_tile_flag<TILE>(a.fold.tile_flag, tile);
         if (s_flag) clear_tile_flag<TILE>(a.fold.tile_flag, tile);
-        if (tile == 0) a.fold.bump[par ^ 1] = 0ull;
     }
     __syncthreads();
     float *__restrict__ row[M::NV];
@@ -565,13 +514,10 @@ __global__ __launch_bounds__(kBlock) void k_update_bdf(UpdateArgs a) {
     for (int j = 0; j < M::NV; j++) row[j] = a.state + (int64_t)j * a.stride;
     const int64_t ld = a.stride;
     const uint32_t step_key = EXT ? drive_step_key(a.ext.seed, step) : 0u;
-    bool spk[ITEMS];
-    int idx[ITEMS];
-    for (int n = 0; n < ITEMS; n++) {
-        idx[n] = tile * TILE + n * kBlock + (int)threadIdx.x;
-        spk[n] = false;
-        if (idx[n] >= a.n) continue;
-        const uint32_t i = (uint32_t)idx[n];
+    const int idx = tile * TILE + (int)threadIdx.x;
+    bool spk = false;
+    if (idx < a.n) {
+        const uint32_t i = (uint32_t)idx;
         float sf[M::NV];
         bdf_load<M, MASK, EXT>(a, row, step, step_key, s_flag, i, sf);
         T S[M::NV];
@@ -587,18 +533,17 @@ __global__ __launch_bounds__(kBlock) void k_update_bdf(UpdateArgs a) {
         c.since_spike = a.last_spike ? (step - 1 - a.last_spike[i]) : (1 << 30);
         int st = a.bdf.st[i];
         integrate_bdf<M, MASK, T>(a.mp, c, (T)a.k.dt, a.bdf, ld, i, st, S);
-        const bool fired = M::spike(a.mp, prev, S);
-        if constexpr (M::kClockOverride) M::clock_override(c, fired, S);
-        if (fired && M::kResetsIntegrator) st = 0;
+        spk = M::spike(a.mp, prev, S);
+        if constexpr (M::kClockOverride) M::clock_override(c, spk, S);
+        if (spk && M::kResetsIntegrator) st = 0;
         a.bdf.st[i] = st;
-        spk[n] = fired;
-        if (fired && a.last_spike) a.last_spike[i] = step;
+        if (spk && a.last_spike) a.last_spike[i] = step;
         float out[M::NV];
 #pragma unroll
         for (int j = 0; j < M::NV; j++) out[j] = (float)S[j];
         bdf_store<M, MASK>(a, row, i, out);
     }
-    tile_spikes_item_major<ITEMS>(a.out, tile, spk, idx);
+    tile_spikes<1, kBdfBlock>(a.out, tile, &spk, &idx);
     clock_finish(a, step);
 }
 
@@ -665,9 +610,10 @@ __global__ __launch_bounds__(kBlock) void k_train(TrainArgs a) {
     if (blockIdx.x == 0 && threadIdx.x == 0) a.ring_cnt[slot] = (int32_t)(e - b);
 }
 
-// Events pushed by the host: order = position in the host's list.  Events
-// handed over in device memory are checked here (target in range, synapse
-// type enabled); one that fails is dropped and sets err bit 8.
+// Events pushed by the host (read from its pinned buffer) or handed over in
+// device memory: order = position in the list.  They are checked here (target
+// in range, synapse type enabled); one that fails is dropped and sets err bit
+// 8 (the host's own were checked when they were queued).
 struct PushEvents {
     const int32_t *tgt;
     const uint8_t *type;
@@ -678,17 +624,18 @@ struct PushEvents {
     uint32_t *err;
 };
 
-template <int PASS>
 __global__ __launch_bounds__(kBlock) void k_fold_push(FoldTarget t, PushEvents e) {
     for (int q = blockIdx.x * kBlock + threadIdx.x; q < e.n; q += gridDim.x * kBlock) {
         const int32_t tg = e.tgt[q];
         const uint32_t ty = e.type[q];
+        const float w = e.w[q];
         if ((uint32_t)tg >= (uint32_t)e.n_tgt || ty > 2u || !((e.mask >> ty) & 1u)) {
-            if (PASS == kCount) atomicOr(e.err, 256u);
+            atomicOr(e.err, 256u);
             continue;
         }
-        const uint64_t key = (uint64_t)ty * (uint64_t)t.stride + (uint64_t)tg;
-        fold_event<PASS>(t, t.par, key, (uint64_t)q, e.w[q]);
+        const uint32_t prev = atomicExch(&t.head[(uint64_t)ty * (uint64_t)t.stride + (uint64_t)tg], (uint32_t)q + 1u);
+        t.node[q] = FoldNode{prev, w};
+        t.tile_flag[(uint32_t)tg / (uint32_t)kFlagTile] = 1u;
     }
 }
 
@@ -769,13 +716,12 @@ __device__ __forceinline__ void stdp_increment(const StdpSyn &s, float *w, int64
 // The order key (ord_key) holds delay, source, chunk and synapse position;
 // within a group the synapse position rises with the source index and then
 // the target index, which is the reference's delivery order in a group.
-template <int PASS, int LANES>
+template <int LANES>
 __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEvents &r, int bid, int nb) {
     __shared__ int64_t s_pref[kMaxDelay * kMaxSources + 1];
     __shared__ int s_slot[kMaxDelay * kMaxSources];
     const int nseg = r.max_delay * r.n_sources;
     const int32_t step = r.step.get();
-    const int par = t.par_by_step ? (step & 1) : t.par;
     const uint32_t rank_lo = (r.rtab && r.skip && r.skip[0] == (uint32_t)step) ? r.skip[1] : 0u;
     for (int g = threadIdx.x; g < nseg; g += kBlock) {
         const int d = g / r.n_sources + 1;
@@ -833,14 +779,14 @@ __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEv
             if (rk < rank_lo || rk >= r.rank_hi) continue;
         }
         double t_arr = 0.0;
-        if (PASS != kCount && src.stdp)
+        if (src.stdp)
             t_arr = (src.poisson ? r.time_ring_p[s_slot[g]] : r.time_ring[s_slot[g]]) + r.delay_s[d];
         for (int64_t q = b + lane; q < e; q += LANES) {
             const uint32_t tt = src.tgt_type[q];
             const uint64_t key =
                 (uint64_t)(tt >> 30) * (uint64_t)t.stride + (uint64_t)(tt & 0x3fffffffu);
-            fold_event<PASS>(t, par, key, ord_hi | (uint64_t)q, src.w[q]);
-            if (PASS != kCount && src.stdp) {
+            fold_event(t, key, ord_hi | (uint64_t)q, src.w[q]);
+            if (src.stdp) {
                 // STDPWeightChange::ApplyPreSynapticSpike (STDPWeightChange.cpp:43-55),
                 // after the event used the weight (PropagatedSpikeGroup.cpp:76-97).
                 // A synapse carries at most one event per step: no other lane
@@ -853,9 +799,9 @@ __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEv
     }
 }
 
-template <int PASS, int LANES>
+template <int LANES>
 __global__ __launch_bounds__(kBlock) void k_fold_ring(FoldTarget t, RingEvents r) {
-    fold_ring_body<PASS, LANES>(t, r, blockIdx.x, gridDim.x);
+    fold_ring_body<LANES>(t, r, blockIdx.x, gridDim.x);
 }
 
 // Compaction of update k's spikes and the fold of the events update k + 1
@@ -867,7 +813,7 @@ __global__ __launch_bounds__(kBlock) void k_compact_fold(CompactArgs c, FoldTarg
                                                          int nb_compact) {
     clock_next_kernel(c);
     if ((int)blockIdx.x < nb_compact) compact_body(c, blockIdx.x, nb_compact);
-    else fold_ring_body<kStatic, LANES>(t, r, blockIdx.x - nb_compact, gridDim.x - nb_compact);
+    else fold_ring_body<LANES>(t, r, blockIdx.x - nb_compact, gridDim.x - nb_compact);
 }
 
 // The same with the event-queue replay of update k's window in the first
@@ -881,7 +827,7 @@ __global__ __launch_bounds__(kBlock) void k_compact_fold_eq(CompactArgs c, FoldT
     const int b = (int)blockIdx.x - 1;
     if (b < 0) eq_body<ITEMS, kEqFusedDelays>(q);
     else if (b < nb_compact) compact_body(c, b, nb_compact);
-    else fold_ring_body<kStatic, LANES>(t, r, b - nb_compact, (int)gridDim.x - 1 - nb_compact);
+    else fold_ring_body<LANES>(t, r, b - nb_compact, (int)gridDim.x - 1 - nb_compact);
 }
 
 // Synapses per (type, target) key of one source, for the fixed segments of

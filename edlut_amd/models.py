@@ -252,9 +252,10 @@ class TimeDrivenNeuronModel_GPU:
             step = int(round(CurrentTime / self._int["step"]))
         n = ctypes.c_int(0)
         C.check(C.lib().edlut_population_update(self._pop, int(step), C.byref(n)))
-        out = np.zeros(max(n.value, 1), np.int32)
-        C.check(C.lib().edlut_population_get_spikes(self._pop, C.ptr(out), len(out)))
-        self._spikes = out[: n.value].copy()
+        out = np.empty(n.value, np.int32)
+        if n.value:
+            C.check(C.lib().edlut_population_get_spikes(self._pop, C.ptr(out), len(out)))
+        self._spikes = out
         return False
 
     def GetInternalSpikeIndexs(self) -> np.ndarray:
