@@ -9,6 +9,7 @@ namespace edl {
 constexpr int kWave = 64;
 constexpr int kBlock = 256;               // threads per update workgroup
 constexpr int kWavesPerBlock = kBlock / kWave;
+constexpr int kGroupAlign = 256;          // grouped populations: groups start on this
 
 // ---------------------------------------------------------------------------
 // Ordered compaction of spiking neuron indices, in two passes without atomics.

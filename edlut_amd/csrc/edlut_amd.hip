@@ -20,6 +20,7 @@
 #include "generate.hpp"
 #include "granule_bdf.hpp"
 #include "kernels.hpp"
+#include "pull.hpp"
 
 using namespace edl;
 
@@ -540,6 +541,11 @@ struct edlut_network {
     // launch shape of the ring fold (set by hand or by the autotuner)
     int fold_lanes = 32;
     int fold_blocks = 512;
+    // grouped populations: incoming lists and spike bits of the pull delivery
+    // (pull.hpp); pull_on: built for the present synapses
+    bool pull_on = false;
+    size_t pull_lds = 0;
+    PullArgs pull{};
     // fixed fold segment of every (type, target) key: prefix of the keys'
     // synapse counts over all sources (rebuilt when sources change)
     uint64_t *seg_off = nullptr;
@@ -1383,16 +1389,21 @@ void launch_compact(hipStream_t st, int32_t *tile_count, int32_t *staging, int n
 }
 
 using RingFoldFn = void (*)(FoldTarget, RingEvents);
-RingFoldFn pick_ring_fold(int lanes) {
+using CompactFoldEqFn = void (*)(CompactArgs, FoldTarget, RingEvents, int, EqArgs);
+// By fold lanes, leaving out the events of pulled groups or not.
+template <bool PULL>
+RingFoldFn ring_fold_fn(int lanes) {
     switch (lanes) {
-        case 8: return k_fold_ring<8>;
-        case 16: return k_fold_ring<16>;
-        case 32: return k_fold_ring<32>;
-        case 64: return k_fold_ring<64>;
+        case 8: return k_fold_ring<8, PULL>;
+        case 16: return k_fold_ring<16, PULL>;
+        case 32: return k_fold_ring<32, PULL>;
+        case 64: return k_fold_ring<64, PULL>;
         default: return nullptr;
     }
 }
-using CompactFoldEqFn = void (*)(CompactArgs, FoldTarget, RingEvents, int, EqArgs);
+RingFoldFn pick_ring_fold(int lanes, bool pull = false) {
+    return pull ? ring_fold_fn<true>(lanes) : ring_fold_fn<false>(lanes);
+}
 template <int ITEMS>
 CompactFoldEqFn compact_fold_eq_fn(int lanes) {
     switch (lanes) {
@@ -1409,19 +1420,23 @@ CompactFoldEqFn pick_compact_fold_eq(int lanes, const EqSim *eq) {
                                           : compact_fold_eq_fn<kEqItems>(lanes);
 }
 using CompactFoldFn = void (*)(CompactArgs, FoldTarget, RingEvents, int);
-CompactFoldFn pick_compact_fold(int lanes) {
+template <bool PULL>
+CompactFoldFn compact_fold_fn(int lanes) {
     switch (lanes) {
-        case 8: return k_compact_fold<8>;
-        case 16: return k_compact_fold<16>;
-        case 32: return k_compact_fold<32>;
-        case 64: return k_compact_fold<64>;
+        case 8: return k_compact_fold<8, PULL>;
+        case 16: return k_compact_fold<16, PULL>;
+        case 32: return k_compact_fold<32, PULL>;
+        case 64: return k_compact_fold<64, PULL>;
         default: return nullptr;
     }
+}
+CompactFoldFn pick_compact_fold(int lanes, bool pull) {
+    return pull ? compact_fold_fn<true>(lanes) : compact_fold_fn<false>(lanes);
 }
 
 // The network-mode fold (one pass into the keys' fixed segments).
 int launch_ring_fold(const FoldTarget &t, hipStream_t st, const RingEvents &re, int lanes, int blocks) {
-    RingFoldFn f = pick_ring_fold(lanes);
+    RingFoldFn f = pick_ring_fold(lanes, re.pulled != nullptr);
     if (!f) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
     hipLaunchKernelGGL(f, dim3(blocks), dim3(kBlock), 0, st, t, re);
     return 0;
@@ -2141,6 +2156,9 @@ int edlut_network_create(edlut_population *pop, int max_delay, edlut_network **o
     return 0;
 }
 
+static void free_pull(edlut_network *n);
+static int clear_pull(edlut_network *n);
+
 int edlut_network_destroy(edlut_network *n) {
     if (!n) return 0;
     if (n->circuit) return fail(EDLUT_E_STATE, "the network belongs to a circuit: destroy the circuit first");
@@ -2161,6 +2179,7 @@ int edlut_network_destroy(edlut_network *n) {
         if (s.from) s.from->links_out--;
     }
     if (n->graph) (void)hipGraphExecDestroy(n->graph);
+    free_pull(n);
     void *dev[] = {n->own_ring_idx, n->own_ring_cnt, n->tile_count, n->staging, n->log_step,
                    n->log_idx, n->log_count, n->d_step, n->d_time, n->d_time_p, n->d_rtab, n->d_skip, n->d_delay_s,
                    n->seg_off, n->clk, n->clk_next};
@@ -2553,8 +2572,19 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
         int rc = launch_ring_fold(ft, p->stream, re, n->fold_lanes, n->fold_blocks);
         if (rc) return rc;
     }
+    if (n->pull_on) {
+        PullArgs pa = n->pull;
+        pa.step = step;
+        hipLaunchKernelGGL(k_pull, dim3((unsigned)pa.n_blocks), dim3(kPullBlock), n->pull_lds, p->stream, pa);
+    }
     UpdateArgs a = make_update_args(p, 0);
     a.step = step;
+    if (n->pull_on) {
+        a.spk_bits = (uint64_t *)n->pull.bits;
+        a.spk_count = n->pull.count;
+        a.ring = n->ring;
+        a.groups = n->pull.groups;
+    }
     a.ext = n->ext;
     a.out = TileOut{n->tile_count, n->staging};
     a.fold = ft;
@@ -2590,7 +2620,7 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
             hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks + 1), dim3(kBlock), 0, p->stream, c, ft, rn, nbc,
                                eq_args(eq, step, 0, 0.0));
         } else {
-            CompactFoldFn f = pick_compact_fold(n->fold_lanes);
+            CompactFoldFn f = pick_compact_fold(n->fold_lanes, re0.pulled != nullptr);
             if (!f) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
             hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks), dim3(kBlock), 0, p->stream, c, ft, rn, nbc);
         }
@@ -2632,6 +2662,11 @@ static RingEvents ring_events(edlut_network *n) {
     re.rtab = (n->eq_on && !n->pop->grouped && !n->sources.empty() && n->eq_rank[0]) ? n->d_rtab : nullptr;
     re.skip = n->d_skip;
     re.rank_hi = 0xffffffffu;
+    if (n->pull_on) {
+        re.pulled = n->pull.mode;
+        re.chunk_group = n->pop->d_chunk_group;
+        re.groups = n->pull.groups;
+    }
     re.exp_lut = n->pop->exp_lut;
     for (int q = 0; q < re.n_sources; q++) {
         const Source &s = n->sources[q];
@@ -2736,6 +2771,166 @@ static int build_segments(edlut_network *n) {
     return 0;
 }
 
+static void free_pull(edlut_network *n) {
+    const PullArgs &a = n->pull;
+    const void *dev[] = {a.blocks, a.ent, a.w, a.slice, a.bits, a.count, a.mode, a.gsize};
+    for (const void *q : dev)
+        if (q) (void)hipFree((void *)q);
+    n->pull = PullArgs{};
+    n->pull_on = false;
+}
+
+// No spike in any slot, every group pushed.
+static int clear_pull(edlut_network *n) {
+    if (!n->pull_on) return 0;
+    const PullArgs &a = n->pull;
+    hipStream_t st = n->pop->stream;
+    HIP_TRY(hipMemsetAsync((void *)a.bits, 0, sizeof(uint32_t) * (size_t)a.ring * a.words_all, st));
+    HIP_TRY(hipMemsetAsync(a.count, 0, sizeof(uint32_t) * (size_t)a.ring * a.groups, st));
+    HIP_TRY(hipMemsetAsync(a.mode, 0, 2 * (size_t)a.groups, st));
+    return 0;
+}
+
+// The incoming lists of a grouped population whose only source is its own
+// recurrent synapses, none of them plastic or between groups, with lists of at
+// most kPullLanesMax synapses and bitmaps that fit the LDS.  Anything else, or
+// too little memory, leaves delivery to the push fold alone.
+static int build_pull(edlut_network *n) {
+    free_pull(n);
+    edlut_population *p = n->pop;
+    if (!p->grouped || n->plastic || n->sources.size() != 1 || !n->sources[0].self || n->sources[0].nsyn == 0) return 0;
+    const Source &s = n->sources[0];
+    const int groups = (int)p->g_size.size(), D = n->max_delay;
+    int64_t lds = 0;
+    for (int32_t g : p->g_size) lds = std::max(lds, ((int64_t)D * ((g + 31) / 32) + 1) * 4);
+    if (lds > kPullLdsMax) return 0;
+    hipStream_t st = p->stream;
+    const int64_t slices = p->stride / kWave, nch = (slices + kScanChunk - 1) / kScanChunk;
+    uint32_t *deg = nullptr, *len = nullptr, *bad = nullptr;
+    int32_t *gstart = nullptr, *gsize = nullptr;
+    int64_t *sums = nullptr, *slice = nullptr;
+    uint32_t *ent = nullptr, *bits = nullptr, *count = nullptr;
+    float *w = nullptr;
+    uint8_t *mode = nullptr;
+    PullBlock *blocks = nullptr;
+    bool ok = true;
+    auto get = [&](auto **q, size_t m) {
+        void *v = nullptr;
+        ok = ok && hipMalloc(&v, std::max<size_t>(m, 1) * sizeof(**q)) == hipSuccess;
+        *q = (std::remove_reference_t<decltype(*q)>)v;
+    };
+    auto done = [&](bool keep) {
+        void *tmp[] = {deg, len, bad, gstart, sums};
+        for (void *q : tmp)
+            if (q) (void)hipFree(q);
+        if (!keep) {
+            void *kept[] = {gsize, slice, ent, bits, count, w, mode, blocks};
+            for (void *q : kept)
+                if (q) (void)hipFree(q);
+            (void)hipGetLastError();
+        }
+        return 0;
+    };
+    std::vector<PullBlock> hb;
+    for (int g = 0; g < groups; g++) {
+        const int32_t padded = (p->g_size[g] + kGroupAlign - 1) / kGroupAlign * kGroupAlign;
+        for (int32_t f = 0; f < padded; f += kPullBlock)
+            hb.push_back(PullBlock{p->g_start[g] + f, std::min(padded - f, (int32_t)kPullBlock), g, p->g_start[g],
+                                   (p->g_size[g] + 31) / 32, p->g_size[g]});
+    }
+    get(&deg, (size_t)p->stride);
+    get(&len, (size_t)slices);
+    get(&bad, 1);
+    get(&gstart, (size_t)groups);
+    get(&gsize, (size_t)groups);
+    get(&sums, (size_t)nch + 1);
+    get(&slice, (size_t)slices + 1);
+    if (!ok) return done(false);
+    ok = hipMemsetAsync(deg, 0, sizeof(uint32_t) * (size_t)p->stride, st) == hipSuccess &&
+         hipMemsetAsync(bad, 0, sizeof(uint32_t), st) == hipSuccess &&
+         hipMemcpyAsync(gstart, p->g_start.data(), sizeof(int32_t) * groups, hipMemcpyHostToDevice, st) == hipSuccess &&
+         hipMemcpyAsync(gsize, p->g_size.data(), sizeof(int32_t) * groups, hipMemcpyHostToDevice, st) == hipSuccess;
+    if (!ok) return done(false);
+    PullBuild b{s.row_ptr, s.tgt_type, s.w, p->n, D, p->d_chunk_group, gstart, gsize, deg, slice, nullptr, nullptr,
+                nullptr, bad};
+    const unsigned rb = (unsigned)std::min<int64_t>(65536, ((int64_t)p->n * D + kBlock - 1) / kBlock);
+    hipLaunchKernelGGL((k_pull_scatter<false>), dim3(rb), dim3(kBlock), 0, st, b);
+    hipLaunchKernelGGL(k_pull_slices, dim3((unsigned)(p->stride / kBlock)), dim3(kBlock), 0, st, deg, p->stride, len);
+    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nch), dim3(kBlock), 0, st, len, slices, sums);
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(kBlock), 0, st, sums, nch);
+    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nch), dim3(kBlock), 0, st, len, slices, (const int64_t *)sums, slice);
+    std::vector<uint32_t> hl((size_t)slices);
+    int64_t rows = 0;
+    uint32_t hbad = 0;
+    ok = hipMemcpyAsync(hl.data(), len, sizeof(uint32_t) * (size_t)slices, hipMemcpyDeviceToHost, st) == hipSuccess &&
+         hipMemcpyAsync(&rows, slice + slices, sizeof(int64_t), hipMemcpyDeviceToHost, st) == hipSuccess &&
+         hipMemcpyAsync(&hbad, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st) == hipSuccess &&
+         hipStreamSynchronize(st) == hipSuccess;
+    if (!ok) {
+        (void)done(false);
+        return fail(EDLUT_E_HIP, "incoming list set-up failed");
+    }
+    const uint32_t longest = *std::max_element(hl.begin(), hl.end());
+    // the keys to sort fill the event buffer (16 bytes per synapse) before any
+    // event does
+    if (hbad || longest > (uint32_t)kPullLanesMax || (uint64_t)rows * kWave * sizeof(uint64_t) > p->b_cap * sizeof(FoldEntry))
+        return done(false);
+    get(&ent, (size_t)rows * kWave);
+    get(&w, (size_t)rows * kWave);
+    get(&bits, (size_t)n->ring * (p->stride / 32));
+    get(&count, (size_t)n->ring * groups);
+    get(&mode, 2 * (size_t)groups);
+    get(&blocks, hb.size());
+    if (!ok) return done(false);
+    int P = 1;
+    while (P < (int)longest) P *= 2;
+    const size_t sort_lds = sizeof(uint64_t) * (size_t)P * kWavesPerBlock;
+    ok = hipMemsetAsync(deg, 0, sizeof(uint32_t) * (size_t)p->stride, st) == hipSuccess &&
+         hipMemcpyAsync(blocks, hb.data(), sizeof(PullBlock) * hb.size(), hipMemcpyHostToDevice, st) == hipSuccess &&
+         hipFuncSetAttribute((const void *)k_pull, hipFuncAttributeMaxDynamicSharedMemorySize, kPullLdsMax) == hipSuccess &&
+         hipFuncSetAttribute((const void *)k_pull_sort, hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)(sizeof(uint64_t) * kPullLanesMax * kWavesPerBlock)) == hipSuccess;
+    if (!ok) {
+        (void)done(false);
+        return fail(EDLUT_E_HIP, "incoming list set-up failed");
+    }
+    b.key = (uint64_t *)p->b_ent;
+    b.ent = ent;
+    b.w_out = w;
+    hipLaunchKernelGGL((k_pull_scatter<true>), dim3(rb), dim3(kBlock), 0, st, b);
+    hipLaunchKernelGGL(k_pull_sort, dim3((unsigned)std::min<int64_t>(16384, p->stride / kWavesPerBlock)), dim3(kBlock),
+                       sort_lds, st, b, p->stride, P);
+    PullArgs &a = n->pull;
+    a.blocks = blocks;
+    a.n_blocks = (int)hb.size();
+    a.groups = groups;
+    a.max_delay = D;
+    a.ring = n->ring;
+    a.ent = ent;
+    a.w = w;
+    a.slice = slice;
+    a.bits = bits;
+    a.words_all = p->stride / 32;
+    a.count = count;
+    a.mode = mode;
+    a.gsize = gsize;
+    a.g_exc = p->state + (int64_t)p->nd * p->stride;
+    a.g_inh = p->state + (int64_t)(p->nd + 1) * p->stride;
+    n->pull_on = true;
+    n->pull_lds = (size_t)lds;
+    const int rc = clear_pull(n);
+    if (!rc)
+        hipLaunchKernelGGL(k_pull_history, dim3(256), dim3(kBlock), 0, st, n->own_ring_idx, n->own_ring_cnt,
+                           (int64_t)p->n, n->ring, p->d_chunk_group, bits, a.words_all, count, groups);
+    const hipError_t e = rc ? hipSuccess : hipStreamSynchronize(st);
+    (void)done(true);
+    if (rc || e != hipSuccess) {
+        free_pull(n);
+        return rc ? rc : fail(EDLUT_E_HIP, "incoming list set-up failed: %s", hipGetErrorString(e));
+    }
+    return 0;
+}
+
 // Everything a run needs before its first step: stale folds dropped, rings
 // cleared when the run does not continue the previous one, segments built,
 // the timing window set.  Returns the update kernel through *fn.
@@ -2755,6 +2950,8 @@ static int run_prepare(edlut_network *n, int64_t first_step, int n_steps, Update
         for (Source &s : n->sources)
             if (!s.from) HIP_TRY(hipMemsetAsync(s.ring_cnt, 0, sizeof(int32_t) * n->ring, p->stream));
         HIP_TRY(hipMemsetAsync(n->own_ring_cnt, 0, sizeof(int32_t) * n->ring, p->stream));
+        const int prc = clear_pull(n);
+        if (prc) return prc;
         int64_t lc[2] = {0, 0};
         HIP_TRY(hipMemcpyAsync(lc, n->log_count, sizeof(lc), hipMemcpyDeviceToHost, p->stream));
         HIP_TRY(hipStreamSynchronize(p->stream));
@@ -2785,7 +2982,7 @@ static int run_prepare(edlut_network *n, int64_t first_step, int n_steps, Update
     if (!*fn) return fail(EDLUT_E_ARG, "no update kernel for this model, integrator and synapse set");
     if (n->seg_dirty) {
         int rc = build_segments(n);
-        if (rc) return rc;
+        if (rc || (rc = build_pull(n))) return rc;
         n->dirty = true;
     }
     p->started = true;
@@ -3495,6 +3692,8 @@ int edlut_network_reset(edlut_network *n) {
         if (s.log_count) HIP_TRY(hipMemsetAsync(s.log_count, 0, 2 * sizeof(int64_t), p->stream));
     }
     HIP_TRY(hipMemsetAsync(n->own_ring_cnt, 0, sizeof(int32_t) * n->ring, p->stream));
+    const int prc = clear_pull(n);
+    if (prc) return prc;
     HIP_TRY(hipMemsetAsync(n->log_count, 0, 2 * sizeof(int64_t), p->stream));
     HIP_TRY(hipMemsetAsync(p->err, 0, sizeof(uint32_t), p->stream));
     HIP_TRY(hipMemsetAsync(n->d_time, 0, sizeof(double) * n->ring, p->stream));
@@ -3619,6 +3818,7 @@ int edlut_network_set_stdp(edlut_network *n, int source, float max_ltp, float ta
         HIP_TRY(hipMemset(p->tile_flag, 0, sizeof(uint32_t) * (p->stride / kFlagTile)));
         n->fold_ready = -1;
     }
+    n->seg_dirty = true;   // plastic synapses are not pulled
     // targets of every synapse -> per-target list of synapse positions
     std::vector<uint32_t> tt((size_t)s.nsyn);
     s.w0.resize((size_t)s.nsyn);

@@ -41,7 +41,6 @@ constexpr int kItems = 4;                    // neurons per thread in the update
 constexpr int kUpdTile = kBlock * kItems;    // neurons per update tile (kItems per thread)
 constexpr int kFlagTile = 512;               // neurons per fold flag (smallest update tile)
 constexpr int kBdfBlock = 512;               // threads, and neurons, of a BDF update tile
-constexpr int kGroupAlign = 256;             // grouped populations: groups start on this
 
 // One queued event of the fold: its order key and weight in one 16-byte
 // entry, so that scattering an event writes one line.
@@ -225,6 +224,11 @@ struct UpdateArgs {
     TileOut out;
     FoldTarget fold;       // ordered input fold of this step (multi-event keys)
     GroupTable grp;        // grouped populations only
+    // grouped populations that can pull (pull.hpp): spike bits and counts per
+    // group by update slot (null: none)
+    uint64_t *spk_bits;    // [ring][stride / 64]
+    uint32_t *spk_count;   // [ring][groups]
+    int ring, groups;
     // timed runs: every workgroup stores its start and end on the device
     // wall clock at clk[((step - clk_first) * gridDim.x + block) * 2 + {0,1}]
     // for steps in [clk_first, clk_first + clk_count) (clk null: untimed)
@@ -442,6 +446,18 @@ __global__ __launch_bounds__(kBlock) void k_update(UpdateArgs a) {
             if (MASK & 2u) __builtin_nontemporal_store(s[n][M::INH], &row[M::INH][i]);
             if (MASK & 4u) __builtin_nontemporal_store(s[n][M::NMDA], &row[M::NMDA][i]);
         }
+    }
+    if (GROUPED && a.spk_bits) {
+        const int slot = step % a.ring;
+        uint32_t total = 0;
+#pragma unroll
+        for (int n = 0; n < ITEMS; n++) {
+            const uint64_t m = __ballot(spk[n]);
+            total += (uint32_t)__popcll(m);
+            if ((threadIdx.x & (kWave - 1)) == 0) a.spk_bits[slot * (a.stride / kWave) + idx[n] / kWave] = m;
+        }
+        if ((threadIdx.x & (kWave - 1)) == 0 && total)
+            atomicAdd(&a.spk_count[(int64_t)slot * a.groups + a.grp.chunk_group[idx[0] / kGroupAlign]], total);
     }
     tile_spikes<ITEMS>(a.out, tile, spk, idx);
     clock_finish(a, step);
@@ -692,6 +708,11 @@ struct RingEvents {
     const RankTab *rtab;
     const uint32_t *skip;
     uint32_t rank_hi;
+    // groups whose events are pulled (pull.hpp), [2][groups] by update parity,
+    // and the group of each kGroupAlign-neuron chunk (null: none)
+    const uint8_t *pulled;
+    const uint32_t *chunk_group;
+    int groups;
 };
 
 // STDPState::SetNewUpdateTime (STDPState.cpp:74-82): both traces decay by
@@ -716,7 +737,8 @@ __device__ __forceinline__ void stdp_increment(const StdpSyn &s, float *w, int64
 // The order key (ord_key) holds delay, source, chunk and synapse position;
 // within a group the synapse position rises with the source index and then
 // the target index, which is the reference's delivery order in a group.
-template <int LANES>
+// PULL: a wave looks 64 items up at once and leaves out the pulled groups'.
+template <int LANES, bool PULL>
 __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEvents &r, int bid, int nb) {
     __shared__ int64_t s_pref[kMaxDelay * kMaxSources + 1];
     __shared__ int s_slot[kMaxDelay * kMaxSources];
@@ -742,6 +764,52 @@ __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEv
     }
     __syncthreads();
     const int64_t n_items = s_pref[nseg];
+    if (PULL) {
+        // a grouped population's own spikes in the canonical order (a single
+        // source, no STDP)
+        const RingSource &src = r.src[0];
+        const uint8_t *pulled = r.pulled + (int64_t)(step & 1) * r.groups;
+        const int wl = threadIdx.x & (kWave - 1);
+        const int64_t wave = (int64_t)bid * kWavesPerBlock + threadIdx.x / kWave;
+        for (int64_t it0 = wave * kWave; it0 < n_items; it0 += (int64_t)nb * kBlock) {
+            const int64_t it = it0 + wl;
+            int64_t b = 0, e = 0;
+            uint64_t ord = 0;
+            if (it < n_items) {
+                int lo = 0, hi = nseg - 1;
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (s_pref[mid] <= it) lo = mid;
+                    else hi = mid - 1;
+                }
+                const int64_t rank = it - s_pref[lo];
+                const int32_t id = src.ring_idx[(int64_t)s_slot[lo] * src.n_src + rank];
+                if (!pulled[r.chunk_group[id / kGroupAlign]]) {
+                    b = src.row_ptr[(int64_t)id * r.max_delay + lo];
+                    e = src.row_ptr[(int64_t)id * r.max_delay + lo + 1];
+                    ord = ord_key(lo + 1, 0, s_pref[lo + 1] - s_pref[lo] >= 1024 ? (uint32_t)(rank >> 10) : 0u, 0);
+                }
+            }
+            uint64_t live = __ballot(b < e);
+            while (live) {
+                // one item per group of LANES lanes
+                int from = -1;
+                for (int u = 0; u < kWave / LANES && live; u++) {
+                    if (wl / LANES == u) from = __builtin_ctzll(live);
+                    live &= live - 1ull;
+                }
+                const int f = from < 0 ? 0 : from;
+                const int64_t fb = __shfl(b, f), fe = __shfl(e, f);
+                const uint64_t fo = __shfl(ord, f);
+                for (int64_t q = fb + wl % LANES; from >= 0 && q < fe; q += LANES) {
+                    const uint32_t tt = src.tgt_type[q];
+                    fold_event(t, (uint64_t)(tt >> 30) * (uint64_t)t.stride + (uint64_t)(tt & 0x3fffffffu),
+                               fo | (uint64_t)q, src.w[q]);
+                }
+            }
+        }
+        return;
+    }
     const int lane = threadIdx.x % LANES;
     const int64_t group = (int64_t)(bid * kBlock + (int)threadIdx.x) / LANES;
     const int64_t n_groups = (int64_t)nb * kBlock / LANES;
@@ -799,21 +867,21 @@ __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEv
     }
 }
 
-template <int LANES>
+template <int LANES, bool PULL = false>
 __global__ __launch_bounds__(kBlock) void k_fold_ring(FoldTarget t, RingEvents r) {
-    fold_ring_body<LANES>(t, r, blockIdx.x, gridDim.x);
+    fold_ring_body<LANES, PULL>(t, r, blockIdx.x, gridDim.x);
 }
 
 // Compaction of update k's spikes and the fold of the events update k + 1
 // consumes, in one launch (network mode without STDP): the fold reads the
 // spike lists of updates <= k - 1 only, and the fold buffers it fills were
 // drained by update k.  Workgroups [0, nb_compact) compact, the rest fold.
-template <int LANES>
+template <int LANES, bool PULL = false>
 __global__ __launch_bounds__(kBlock) void k_compact_fold(CompactArgs c, FoldTarget t, RingEvents r,
                                                          int nb_compact) {
     clock_next_kernel(c);
     if ((int)blockIdx.x < nb_compact) compact_body(c, blockIdx.x, nb_compact);
-    else fold_ring_body<LANES>(t, r, blockIdx.x - nb_compact, gridDim.x - nb_compact);
+    else fold_ring_body<LANES, PULL>(t, r, blockIdx.x - nb_compact, gridDim.x - nb_compact);
 }
 
 // The same with the event-queue replay of update k's window in the first
@@ -827,7 +895,7 @@ __global__ __launch_bounds__(kBlock) void k_compact_fold_eq(CompactArgs c, FoldT
     const int b = (int)blockIdx.x - 1;
     if (b < 0) eq_body<ITEMS, kEqFusedDelays>(q);
     else if (b < nb_compact) compact_body(c, b, nb_compact);
-    else fold_ring_body<LANES>(t, r, b - nb_compact, (int)gridDim.x - 1 - nb_compact);
+    else fold_ring_body<LANES, false>(t, r, b - nb_compact, (int)gridDim.x - 1 - nb_compact);
 }
 
 // Synapses per (type, target) key of one source, for the fixed segments of
