@@ -648,6 +648,7 @@ namespace {
 // PoissonGeneratorDeviceVector samples every 0.1f ms of its millisecond time
 // scale: 0.1f / 1000.0f in float (PoissonGeneratorDeviceVector.cpp:26,137).
 inline double poisson_step_s() { return (double)(0.1f / 1000.0f); }
+inline int poisson_tiles(const Source &s) { return (int)((s.n + kBlock - 1) / kBlock); }
 
 int64_t g_train_seq = 0;   // load order of input spikes across spike trains
 
@@ -1023,8 +1024,16 @@ int eq_resume(EqSim *S, int64_t first, int n_steps, double stop, hipStream_t st)
         E.in_loaded = hi;
         changed = true;
     }
-    // the populations' update tiles (their layout follows the launch shape)
+    // the update's tiles: the Poisson devices' and the populations' (whose
+    // layout follows the launch shape)
     for (EqHostEm &E : S->em) {
+        if (E.kind == kEqPoisson) {
+            const Source &s = E.copies[0].first->sources[(size_t)E.copies[0].second];
+            E.dev.tile_count = s.tile_count;
+            E.dev.staging = s.staging;
+            E.dev.n_tiles = poisson_tiles(s);
+            E.dev.tile_size = kBlock;
+        }
         if (E.kind != kEqPop) continue;
         edlut_population *p = E.net->pop;
         E.dev.tile_count = E.net->tile_count;
@@ -2526,52 +2535,89 @@ static FoldTarget net_fold_target(const edlut_network *n) {
     return ft;
 }
 
-// eq: the replayed event queue to advance after this step (a network that
-// runs alone), or null.
-static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingEvents &re0,
-                        bool fold_done, bool *fused, const EqSim *eq = nullptr) {
-    edlut_population *p = n->pop;
-    if (n->plastic)
-        hipLaunchKernelGGL(k_tick, dim3(1), dim3(64), 0, p->stream, step, n->d_time, n->d_time_p, n->ring,
-                           (double)p->dt_s, poisson_step_s());
-    // Poisson devices fire at update k (their spikes feed later updates).
-    for (Source &s : n->sources) {
-        if (s.self || s.from) continue;
-        if (s.train) {
-            TrainArgs ta;
-            ta.ptr = s.train_ptr;
-            ta.idx = s.train_idx;
-            ta.n_steps = s.train_steps;
-            ta.ring_idx = s.ring_idx;
-            ta.ring_cnt = s.ring_cnt;
-            ta.n_src = s.n;
-            ta.ring = n->ring;
-            ta.step = step;
-            hipLaunchKernelGGL(k_train, dim3(s.train_blocks), dim3(kBlock), 0, p->stream, ta);
-            continue;
+// A step's launches hold a few roles each; full ones go out at once.
+static void launch_head(const StepHead &h, hipStream_t st) {
+    int nb = h.n_tick;
+    for (int i = 0; i < h.n_train; i++) nb += h.train_blocks[i];
+    for (int i = 0; i < h.n_poisson; i++) nb += h.poisson[i].n_tiles;
+    for (int i = 0; i < h.n_fold; i++) nb += h.fold[i].blocks;
+    if (nb > 0) hipLaunchKernelGGL(k_step_head, dim3(nb), dim3(kBlock), 0, st, h);
+}
+static void launch_tail(const StepTail &t, const EqSim *eq, const EqArgs &q, hipStream_t st) {
+    int nb = eq ? 1 : 0;
+    for (int i = 0; i < t.n_list; i++) nb += t.list_blocks[i];
+    for (int i = 0; i < t.n_fold; i++) nb += t.fold[i].blocks;
+    if (nb == 0) return;
+    if (!eq) hipLaunchKernelGGL(k_step_tail<0>, dim3(nb), dim3(kBlock), 0, st, t, q);
+    else if (eq->in_flight <= kEqFusedItems)
+        hipLaunchKernelGGL(k_step_tail<kEqFusedItems>, dim3(nb), dim3(kBlock), 0, st, t, q);
+    else hipLaunchKernelGGL(k_step_tail<kEqItems>, dim3(nb), dim3(kBlock), 0, st, t, q);
+}
+
+static bool folds_ahead(const edlut_network *n, const RingEvents &re) { return re.n_sources > 0 && !n->plastic; }
+
+// The clocks, input devices and plastic folds of update k of every network.
+static int enqueue_head(const std::vector<edlut_network *> &nets, StepRef step, const std::vector<RingEvents> &res,
+                        hipStream_t st) {
+    StepHead h;
+    std::memset(&h, 0, sizeof(h));
+    h.step = step;
+    auto flush = [&]() {
+        launch_head(h, st);
+        h.n_tick = h.n_train = h.n_poisson = h.n_fold = 0;
+    };
+    for (size_t j = 0; j < nets.size(); j++) {
+        edlut_network *n = nets[j];
+        if (n->plastic) {
+            if (h.n_tick == kHeadRoles) flush();
+            h.tick[h.n_tick++] = TickArgs{n->d_time, n->d_time_p, n->ring, (double)n->pop->dt_s, poisson_step_s()};
         }
-        PoissonArgs pa;
-        std::memset(&pa, 0, sizeof(pa));
-        pa.lcg = s.lcg;
-        pa.n = (int)s.n;
-        pa.n_tiles = (int)((s.n + kBlock - 1) / kBlock);
-        pa.rate = s.rate;
-        pa.rates = s.rates;
-        pa.step_s = poisson_step_s();
-        pa.out = TileOut{s.tile_count, s.staging};
-        hipLaunchKernelGGL(k_poisson, dim3(pa.n_tiles), dim3(kBlock), 0, p->stream, pa);
-        launch_compact(p->stream, s.tile_count, s.staging, pa.n_tiles, kBlock, s.ring_idx, s.ring_cnt,
-                       n->ring, s.n, s.log_step, s.log_idx, s.log_count, s.log_cap, p->err, step);
+        // Poisson devices fire at update k (their spikes feed later updates).
+        for (Source &s : n->sources) {
+            if (s.self || s.from) continue;
+            if (s.train) {
+                if (h.n_train == kHeadRoles) flush();
+                TrainArgs &ta = h.train[h.n_train];
+                ta.ptr = s.train_ptr;
+                ta.idx = s.train_idx;
+                ta.n_steps = s.train_steps;
+                ta.ring_idx = s.ring_idx;
+                ta.ring_cnt = s.ring_cnt;
+                ta.n_src = s.n;
+                ta.ring = n->ring;
+                ta.step = step;
+                h.train_blocks[h.n_train++] = s.train_blocks;
+                continue;
+            }
+            if (h.n_poisson == kHeadRoles) flush();
+            PoissonArgs &pa = h.poisson[h.n_poisson++];
+            pa.lcg = s.lcg;
+            pa.n = (int)s.n;
+            pa.n_tiles = poisson_tiles(s);
+            pa.rate = s.rate;
+            pa.rates = s.rates;
+            pa.step_s = poisson_step_s();
+            pa.out = TileOut{s.tile_count, s.staging};
+        }
+        // STDP orders the post-synaptic learning of update k before the
+        // arrivals of update k + 1, so plastic networks fold in their own step.
+        if (res[j].n_sources > 0 && n->plastic) {
+            if (h.n_fold == kHeadFolds) flush();
+            FoldRole &f = h.fold[h.n_fold++];
+            f.target = net_fold_target(n);
+            f.events = res[j];
+            f.events.step = step;
+            f.blocks = n->fold_blocks;
+            f.lanes = n->fold_lanes;
+        }
     }
-    // Deliver the events consumed by update k into their keys' segments.
-    FoldTarget ft = net_fold_target(n);
-    const bool ring = re0.n_sources > 0;
-    if (ring && !fold_done) {
-        RingEvents re = re0;
-        re.step = step;
-        int rc = launch_ring_fold(ft, p->stream, re, n->fold_lanes, n->fold_blocks);
-        if (rc) return rc;
-    }
+    flush();
+    return 0;
+}
+
+// The update kernel of one network (with the pulled events of a grouped one).
+static void enqueue_update(edlut_network *n, StepRef step, UpdateFn fn) {
+    edlut_population *p = n->pop;
     if (n->pull_on) {
         PullArgs pa = n->pull;
         pa.step = step;
@@ -2587,8 +2633,7 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
     }
     a.ext = n->ext;
     a.out = TileOut{n->tile_count, n->staging};
-    a.fold = ft;
-    const int tiles = p->update_tiles();
+    a.fold = net_fold_target(n);
     if (n->clk) {
         // timed run: every workgroup stamps its start and end
         a.clk = n->clk;
@@ -2596,7 +2641,11 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
         a.clk_count = (int32_t)n->clk_count;
     }
     hipLaunchKernelGGL(fn, dim3(p->update_blocks()), dim3(p->update_threads()), update_lds_bytes(p), p->stream, a);
-    CompactArgs c = compact_args(n->tile_count, n->staging, tiles, p->tile_size(), n->own_ring_idx,
+}
+
+static CompactArgs net_compact_args(edlut_network *n, StepRef step) {
+    edlut_population *p = n->pop;
+    CompactArgs c = compact_args(n->tile_count, n->staging, p->update_tiles(), p->tile_size(), n->own_ring_idx,
                                  n->own_ring_cnt, n->ring, p->n, n->log_cap ? n->log_step : nullptr,
                                  n->log_cap ? n->log_idx : nullptr, n->log_count, n->log_cap, p->err, step);
     if (n->clk) {
@@ -2604,49 +2653,139 @@ static int enqueue_step(edlut_network *n, StepRef step, UpdateFn fn, const RingE
         c.clk_first = (int32_t)n->clk_first;
         c.clk_count = (int32_t)n->clk_count;
     }
-    const int nbc = compact_blocks(tiles);
-    // STDP orders the post-synaptic learning of update k before the arrivals
-    // of update k + 1, so plastic networks fold in their own step.
-    *fused = ring && !n->plastic;
-    // the event-queue replay of this update's window runs in the compaction
-    // kernel's last workgroup when its sizes fit there
-    const bool eq_fused = *fused && eq && eq->max_delay <= kEqFusedDelays;
-    if (*fused) {
-        RingEvents rn = re0;
-        rn.step = StepRef{step.ptr, step.imm + 1};
-        if (eq_fused) {
+    return c;
+}
+
+// A timed network of a circuit compacts in a kernel of its own, whose start
+// ends its update kernel's time.
+static bool own_list(const std::vector<edlut_network *> &nets, size_t j) { return nets.size() > 1 && nets[j]->clk; }
+
+// The lists of update k of every network and device, the folds of update
+// k + 1 and, with `eq`, the event-queue replay.  A network alone without
+// Poisson devices or plastic synapses has one list and one fold, in the
+// kernel of its lanes.
+static int enqueue_tail(const std::vector<edlut_network *> &nets, StepRef step, const std::vector<RingEvents> &res,
+                        const EqSim *eq, hipStream_t st) {
+    const StepRef next{step.ptr, step.imm + 1};
+    bool devices = false;
+    for (const Source &s : nets[0]->sources) devices = devices || (!s.self && !s.from && !s.train);
+    if (nets.size() == 1 && !devices && (folds_ahead(nets[0], res[0]) || !eq)) {
+        edlut_network *n = nets[0];
+        const CompactArgs c = net_compact_args(n, step);
+        const int nbc = compact_blocks(c.n_tiles);
+        if (!folds_ahead(n, res[0])) {
+            hipLaunchKernelGGL(k_compact, dim3(nbc), dim3(kBlock), 0, st, c);
+            return 0;
+        }
+        RingEvents rn = res[0];
+        rn.step = next;
+        if (eq) {
             CompactFoldEqFn f = pick_compact_fold_eq(n->fold_lanes, eq);
             if (!f) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
-            hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks + 1), dim3(kBlock), 0, p->stream, c, ft, rn, nbc,
-                               eq_args(eq, step, 0, 0.0));
+            hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks + 1), dim3(kBlock), 0, st, c, net_fold_target(n), rn,
+                               nbc, eq_args(eq, step, 0, 0.0));
         } else {
-            CompactFoldFn f = pick_compact_fold(n->fold_lanes, re0.pulled != nullptr);
+            CompactFoldFn f = pick_compact_fold(n->fold_lanes, rn.pulled != nullptr);
             if (!f) return fail(EDLUT_E_ARG, "fold lanes must be 8, 16, 32 or 64");
-            hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks), dim3(kBlock), 0, p->stream, c, ft, rn, nbc);
+            hipLaunchKernelGGL(f, dim3(nbc + n->fold_blocks), dim3(kBlock), 0, st, c, net_fold_target(n), rn, nbc);
         }
-    } else {
-        hipLaunchKernelGGL(k_compact, dim3(nbc), dim3(kBlock), 0, p->stream, c);
+        return 0;
     }
-    // post-synaptic learning of the neurons that fired at this update
-    for (Source &s : n->sources) {
-        if (!s.stdp) continue;
-        StdpPostArgs pa;
-        pa.spk_idx = n->own_ring_idx;
-        pa.spk_cnt = n->own_ring_cnt;
-        pa.slot_len = p->n;
-        pa.ring = n->ring;
-        pa.step = step;
-        pa.in_ptr = s.in_ptr;
-        pa.in_syn = s.in_syn;
-        pa.chunks = (int)((s.in_max + kWave - 1) / kWave);
-        if (pa.chunks < 1) pa.chunks = 1;
-        pa.w = s.w;
-        pa.syn = s.syn;
-        pa.time_ring = n->d_time;
-        pa.exp_lut = p->exp_lut;
-        hipLaunchKernelGGL(k_stdp_post, dim3(64), dim3(kBlock), 0, p->stream, pa);
+    StepTail t;
+    std::memset(&t, 0, sizeof(t));
+    EqArgs q;
+    std::memset(&q, 0, sizeof(q));
+    if (eq) q = eq_args(eq, step, 0, 0.0);
+    auto flush = [&]() {
+        launch_tail(t, eq, q, st);
+        eq = nullptr;   // in the first launch
+        t.n_list = t.n_fold = 0;
+    };
+    auto list = [&](const CompactArgs &c) {
+        if (t.n_list == kTailLists) flush();
+        t.list[t.n_list] = c;
+        t.list_blocks[t.n_list++] = compact_blocks(c.n_tiles);
+    };
+    for (size_t j = 0; j < nets.size(); j++) {
+        edlut_network *n = nets[j];
+        for (Source &s : n->sources) {
+            if (s.self || s.from || s.train) continue;
+            list(compact_args(s.tile_count, s.staging, poisson_tiles(s), kBlock, s.ring_idx, s.ring_cnt, n->ring, s.n,
+                              s.log_step, s.log_idx, s.log_count, s.log_cap, n->pop->err, step));
+        }
+        if (!own_list(nets, j)) list(net_compact_args(n, step));
+        if (folds_ahead(n, res[j])) {
+            if (t.n_fold == kTailFolds) flush();
+            FoldRole &f = t.fold[t.n_fold++];
+            f.target = net_fold_target(n);
+            f.events = res[j];
+            f.events.step = next;
+            f.blocks = n->fold_blocks;
+            f.lanes = n->fold_lanes;
+        }
     }
-    if (eq && !eq_fused) hipLaunchKernelGGL(k_eventq, dim3(1), dim3(kBlock), 0, p->stream, eq_args(eq, step, 0, 0.0));
+    flush();
+    return 0;
+}
+
+// Post-synaptic learning of the neurons that fired at update k.
+static void enqueue_post(const std::vector<edlut_network *> &nets, StepRef step, hipStream_t st) {
+    StepPost t;
+    std::memset(&t, 0, sizeof(t));
+    t.blocks = 64;
+    auto flush = [&]() {
+        if (t.n_post > 0) hipLaunchKernelGGL(k_step_post, dim3(t.n_post * t.blocks), dim3(kBlock), 0, st, t);
+        t.n_post = 0;
+    };
+    for (edlut_network *n : nets)
+        for (Source &s : n->sources) {
+            if (!s.stdp) continue;
+            if (t.n_post == kPostRoles) flush();
+            StdpPostArgs &pa = t.post[t.n_post++];
+            pa.spk_idx = n->own_ring_idx;
+            pa.spk_cnt = n->own_ring_cnt;
+            pa.slot_len = n->pop->n;
+            pa.ring = n->ring;
+            pa.step = step;
+            pa.in_ptr = s.in_ptr;
+            pa.in_syn = s.in_syn;
+            pa.chunks = (int)((s.in_max + kWave - 1) / kWave);
+            if (pa.chunks < 1) pa.chunks = 1;
+            pa.w = s.w;
+            pa.syn = s.syn;
+            pa.time_ring = n->d_time;
+            pa.exp_lut = n->pop->exp_lut;
+        }
+    flush();
+}
+
+// One update of a network alone or of a circuit's members in lockstep:
+// fold_done[j] says whether network j's events of this update are folded
+// already, and is set to whether those of the next one are.  The replay of
+// this update's window runs in the tail when its sizes fit there.
+static int enqueue_step(const std::vector<edlut_network *> &nets, StepRef step, const std::vector<UpdateFn> &fns,
+                        const std::vector<RingEvents> &res, std::vector<bool> &fold_done, const EqSim *eq,
+                        hipStream_t st) {
+    int rc = enqueue_head(nets, step, res, st);
+    if (rc) return rc;
+    for (size_t j = 0; j < nets.size(); j++) {
+        if (!folds_ahead(nets[j], res[j]) || fold_done[j]) continue;
+        RingEvents re = res[j];
+        re.step = step;
+        if ((rc = launch_ring_fold(net_fold_target(nets[j]), st, re, nets[j]->fold_lanes, nets[j]->fold_blocks)))
+            return rc;
+    }
+    for (size_t j = 0; j < nets.size(); j++) {
+        enqueue_update(nets[j], step, fns[j]);
+        if (!own_list(nets, j)) continue;
+        const CompactArgs c = net_compact_args(nets[j], step);
+        hipLaunchKernelGGL(k_compact, dim3(compact_blocks(c.n_tiles)), dim3(kBlock), 0, st, c);
+    }
+    const bool eq_fused = eq && eq->max_delay <= kEqFusedDelays;
+    if ((rc = enqueue_tail(nets, step, res, eq_fused ? eq : nullptr, st))) return rc;
+    enqueue_post(nets, step, st);
+    if (eq && !eq_fused) hipLaunchKernelGGL(k_eventq, dim3(1), dim3(kBlock), 0, st, eq_args(eq, step, 0, 0.0));
+    for (size_t j = 0; j < nets.size(); j++) fold_done[j] = folds_ahead(nets[j], res[j]);
     return 0;
 }
 
@@ -2714,11 +2853,10 @@ static int build_graph(edlut_network *n, UpdateFn fn) {
     int rc = 0;
     // the fold of each captured step ran in the step before it when fused
     // (the run launches the fold of the chunk's first step when needed)
-    const bool will_fuse = re.n_sources > 0 && !n->plastic;
-    bool fused = will_fuse;
+    std::vector<bool> fold_done{folds_ahead(n, re)};
     for (int i = 0; i < kGraphChunk && rc == 0; i++)
-        rc = enqueue_step(n, StepRef{n->d_step, i}, fn, re, fused, &fused, net_eq(n));
-    n->graph_fused = will_fuse;
+        rc = enqueue_step({n}, StepRef{n->d_step, i}, {fn}, {re}, fold_done, net_eq(n), p->stream);
+    n->graph_fused = folds_ahead(n, re);
     hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(64), 0, p->stream, n->d_step, (int32_t)kGraphChunk);
     hipError_t e = hipStreamEndCapture(p->stream, &g);
     if (rc) {
@@ -3091,10 +3229,10 @@ int edlut_network_run(edlut_network *n, int64_t first_step, int n_steps) {
         n->fold_ready = n->graph_fused ? k : -1;
     }
     for (; k < first_step + n_steps; k++) {
-        bool fused = false;
-        if ((rc = enqueue_step(n, StepRef{nullptr, (int32_t)k}, fn, re, n->fold_ready == k, &fused, net_eq(n))))
+        std::vector<bool> fold_done{n->fold_ready == k};
+        if ((rc = enqueue_step({n}, StepRef{nullptr, (int32_t)k}, {fn}, {re}, fold_done, net_eq(n), p->stream)))
             return rc;
-        n->fold_ready = fused ? k + 1 : -1;
+        n->fold_ready = fold_done[0] ? k + 1 : -1;
     }
     HIP_TRY(hipGetLastError());
     run_finish(n, first_step, n_steps);
@@ -3194,19 +3332,13 @@ static int build_circuit_graph(edlut_circuit *c, const std::vector<UpdateFn> &fn
         c->graph = nullptr;
     }
     const size_t m = c->nets.size();
-    std::vector<bool> fused(m);
-    for (size_t j = 0; j < m; j++) fused[j] = res[j].n_sources > 0 && !c->nets[j]->plastic;
+    std::vector<bool> fold_done(m);
+    for (size_t j = 0; j < m; j++) fold_done[j] = folds_ahead(c->nets[j], res[j]);
     hipGraph_t g = nullptr;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     int rc = 0;
-    for (int i = 0; i < kGraphChunk && rc == 0; i++) {
-        for (size_t j = 0; j < m && rc == 0; j++) {
-            bool f = fused[j];
-            rc = enqueue_step(c->nets[j], StepRef{c->d_step, i}, fns[j], res[j], f, &f);
-            fused[j] = f;
-        }
-        if (eq) hipLaunchKernelGGL(k_eventq, dim3(1), dim3(kBlock), 0, c->stream, eq_args(eq, StepRef{c->d_step, i}, 0, 0.0));
-    }
+    for (int i = 0; i < kGraphChunk && rc == 0; i++)
+        rc = enqueue_step(c->nets, StepRef{c->d_step, i}, fns, res, fold_done, eq, c->stream);
     hipLaunchKernelGGL(k_advance_step, dim3(1), dim3(64), 0, c->stream, c->d_step, (int32_t)kGraphChunk);
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (rc) {
@@ -3219,7 +3351,7 @@ static int build_circuit_graph(edlut_circuit *c, const std::vector<UpdateFn> &fn
     if (e != hipSuccess) return fail(EDLUT_E_HIP, "graph instantiation failed");
     for (size_t j = 0; j < m; j++) {
         edlut_network *n = c->nets[j];
-        n->graph_fused = res[j].n_sources > 0 && !n->plastic;
+        n->graph_fused = folds_ahead(n, res[j]);
         // a network's own graph is stale once it has run inside the circuit
         if (n->graph) (void)hipGraphExecDestroy(n->graph);
         n->graph = nullptr;
@@ -3290,14 +3422,10 @@ int edlut_circuit_run(edlut_circuit *c, int64_t first_step, int n_steps) {
         for (size_t j = 0; j < m; j++) c->nets[j]->fold_ready = c->nets[j]->graph_fused ? k : -1;
     }
     for (; k < first_step + n_steps; k++) {
-        for (size_t j = 0; j < m; j++) {
-            edlut_network *n = c->nets[j];
-            bool fused = false;
-            if ((rc = enqueue_step(n, StepRef{nullptr, (int32_t)k}, fns[j], res[j], n->fold_ready == k, &fused)))
-                return rc;
-            n->fold_ready = fused ? k + 1 : -1;
-        }
-        if (eq) hipLaunchKernelGGL(k_eventq, dim3(1), dim3(kBlock), 0, c->stream, eq_args(eq, StepRef{nullptr, (int32_t)k}, 0, 0.0));
+        std::vector<bool> fold_done(m);
+        for (size_t j = 0; j < m; j++) fold_done[j] = c->nets[j]->fold_ready == k;
+        if ((rc = enqueue_step(c->nets, StepRef{nullptr, (int32_t)k}, fns, res, fold_done, eq, c->stream))) return rc;
+        for (size_t j = 0; j < m; j++) c->nets[j]->fold_ready = fold_done[j] ? k + 1 : -1;
     }
     HIP_TRY(hipGetLastError());
     for (size_t j = 0; j < m; j++) run_finish(c->nets[j], first_step, n_steps);

@@ -14,10 +14,10 @@
 // (Simulation.cpp:322-373): a stop event at the stop time, then events until
 // it leaves.
 //
-// k_eventq replays exactly these heap operations, once per update k, after
-// the spikes of update k are compacted: it pops the events that reach the
-// populations between update k and update k + 1 and gives each group (or
-// propagated input spike) its rank in that window.  The fold of update k + 1
+// eq_body replays exactly these heap operations, once per update k, from the
+// spikes of update k (in the update's tiles or the compacted lists): it pops
+// the events that reach the populations between update k and update k + 1 and
+// gives each group (or propagated input spike) its rank in that window.  The fold of update k + 1
 // sorts each target's events by (rank, synapse), which is the reference's
 // delivery order.  The heap holds only keys and small payloads; one wave
 // runs its operations lane-parallel, after the workgroup has counted the
@@ -779,7 +779,7 @@ constexpr int kEqItems = 4096;
 constexpr int kEqFusedItems = 1024;
 constexpr int kEqFusedDelays = 64;
 
-// The replay as a kernel of its own (circuits, plastic networks, resuming calls).
+// The replay as a kernel of its own (delays beyond kEqFusedDelays, resuming calls).
 __global__ __launch_bounds__(kBlock) void k_eventq(EqArgs a) { eq_body<kEqItems, kMaxDelayEq>(a); }
 
 }  // namespace edl

@@ -3,7 +3,7 @@
 //   k_update     one step of every neuron: optional external drive, ODE step,
 //                conductance decay, threshold/reset, NaN reset and ordered
 //                spike compaction (one fused pass over the SoA state).
-//   k_poisson    one step of a Poisson generator device (per-source LCG).
+//   k_step_*     a step's Poisson devices, trains, lists, folds and learning, launched together.
 //   k_fold_*     ordered conductance accumulation of a step's input events.
 #pragma once
 #include <type_traits>
@@ -578,8 +578,7 @@ struct PoissonArgs {
     TileOut out;
 };
 
-__global__ __launch_bounds__(kBlock) void k_poisson(PoissonArgs a) {
-    const int tile = blockIdx.x;
+__device__ __forceinline__ void poisson_body(const PoissonArgs &a, int tile) {
     bool spk[1] = {false};
     int idx[1] = {tile * kBlock + (int)threadIdx.x};
     const int i = idx[0];
@@ -612,7 +611,7 @@ struct TrainArgs {
     StepRef step;
 };
 
-__global__ __launch_bounds__(kBlock) void k_train(TrainArgs a) {
+__device__ __forceinline__ void train_body(const TrainArgs &a, int bid, int nb) {
     const int32_t k = a.step.get();
     const int slot = k % a.ring;
     int64_t b = 0, e = 0;
@@ -621,9 +620,8 @@ __global__ __launch_bounds__(kBlock) void k_train(TrainArgs a) {
         e = a.ptr[k];
     }
     int32_t *out = a.ring_idx + (int64_t)slot * a.n_src;
-    for (int64_t j = b + (int64_t)blockIdx.x * kBlock + threadIdx.x; j < e; j += (int64_t)gridDim.x * kBlock)
-        out[j - b] = a.idx[j];
-    if (blockIdx.x == 0 && threadIdx.x == 0) a.ring_cnt[slot] = (int32_t)(e - b);
+    for (int64_t j = b + (int64_t)bid * kBlock + threadIdx.x; j < e; j += (int64_t)nb * kBlock) out[j - b] = a.idx[j];
+    if (bid == 0 && threadIdx.x == 0) a.ring_cnt[slot] = (int32_t)(e - b);
 }
 
 // Events pushed by the host (read from its pinned buffer) or handed over in
@@ -738,10 +736,22 @@ __device__ __forceinline__ void stdp_increment(const StdpSyn &s, float *w, int64
 // within a group the synapse position rises with the source index and then
 // the target index, which is the reference's delivery order in a group.
 // PULL: a wave looks 64 items up at once and leaves out the pulled groups'.
-template <int LANES, bool PULL>
-__device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEvents &r, int bid, int nb) {
-    __shared__ int64_t s_pref[kMaxDelay * kMaxSources + 1];
-    __shared__ int s_slot[kMaxDelay * kMaxSources];
+// FIXED lanes (a power of two) or, where it is 0, `lanes`.
+struct FoldLds {
+    int64_t pref[kMaxDelay * kMaxSources + 1];
+    int slot[kMaxDelay * kMaxSources];
+};
+__device__ __forceinline__ FoldLds &fold_lds() {
+    __shared__ FoldLds s;
+    return s;
+}
+template <int FIXED, bool PULL>
+__device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEvents &r, int bid, int nb,
+                                               int lanes = FIXED) {
+    const int LANES = FIXED > 0 ? FIXED : lanes;
+    const int shift = __builtin_ctz((unsigned)LANES);
+    int64_t *const s_pref = fold_lds().pref;
+    int *const s_slot = fold_lds().slot;
     const int nseg = r.max_delay * r.n_sources;
     const int32_t step = r.step.get();
     const uint32_t rank_lo = (r.rtab && r.skip && r.skip[0] == (uint32_t)step) ? r.skip[1] : 0u;
@@ -794,14 +804,14 @@ __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEv
             while (live) {
                 // one item per group of LANES lanes
                 int from = -1;
-                for (int u = 0; u < kWave / LANES && live; u++) {
-                    if (wl / LANES == u) from = __builtin_ctzll(live);
+                for (int u = 0; u < (kWave >> shift) && live; u++) {
+                    if ((wl >> shift) == u) from = __builtin_ctzll(live);
                     live &= live - 1ull;
                 }
                 const int f = from < 0 ? 0 : from;
                 const int64_t fb = __shfl(b, f), fe = __shfl(e, f);
                 const uint64_t fo = __shfl(ord, f);
-                for (int64_t q = fb + wl % LANES; from >= 0 && q < fe; q += LANES) {
+                for (int64_t q = fb + (wl & (LANES - 1)); from >= 0 && q < fe; q += LANES) {
                     const uint32_t tt = src.tgt_type[q];
                     fold_event(t, (uint64_t)(tt >> 30) * (uint64_t)t.stride + (uint64_t)(tt & 0x3fffffffu),
                                fo | (uint64_t)q, src.w[q]);
@@ -810,9 +820,9 @@ __device__ __forceinline__ void fold_ring_body(const FoldTarget &t, const RingEv
         }
         return;
     }
-    const int lane = threadIdx.x % LANES;
-    const int64_t group = (int64_t)(bid * kBlock + (int)threadIdx.x) / LANES;
-    const int64_t n_groups = (int64_t)nb * kBlock / LANES;
+    const int lane = (int)threadIdx.x & (LANES - 1);
+    const int64_t group = (int64_t)(bid * kBlock + (int)threadIdx.x) >> shift;
+    const int64_t n_groups = (int64_t)nb * kBlock >> shift;
     for (int64_t it = group; it < n_items; it += n_groups) {
         // last segment g with s_pref[g] <= it (segments may be empty)
         int lo = 0, hi = nseg - 1;
@@ -936,15 +946,15 @@ struct StdpPostArgs {
 // item is one wave-sized chunk of one neuron's list, so a neuron with 2,000
 // inputs is spread over 32 waves rather than walked by one; the synapses are
 // distinct, so the order of their updates does not matter.
-__global__ __launch_bounds__(kBlock) void k_stdp_post(StdpPostArgs a) {
+__device__ __forceinline__ void stdp_post_body(const StdpPostArgs &a, int bid, int nb) {
     const int32_t step = a.step.get();
     const int slot = step % a.ring;
     const int64_t n = a.spk_cnt[slot];
     const int32_t *ids = a.spk_idx + (int64_t)slot * a.slot_len;
     const double tk = a.time_ring[slot];
     const int lane = threadIdx.x % kWave;
-    const int64_t wave = (int64_t)(blockIdx.x * kBlock + threadIdx.x) / kWave;
-    const int64_t n_waves = (int64_t)gridDim.x * kBlock / kWave;
+    const int64_t wave = (int64_t)(bid * kBlock + (int)threadIdx.x) / kWave;
+    const int64_t n_waves = (int64_t)nb * kBlock / kWave;
     for (int64_t it = wave; it < n * a.chunks; it += n_waves) {
         const int32_t i = ids[it / a.chunks];
         const int64_t x = a.in_ptr[i] + (it % a.chunks) * kWave + lane;
@@ -958,14 +968,143 @@ __global__ __launch_bounds__(kBlock) void k_stdp_post(StdpPostArgs a) {
 }
 
 // Update time of step k: t_k = t_{k-1} + double(float dt), kept per ring slot
-// (TimeEventUpdateNeurons.cpp:78).  First node of a step of a plastic network.
-// The Poisson devices' clock advances by their own step in a second ring.
-__global__ void k_tick(StepRef step, double *time_ring, double *time_ring_p, int ring, double dt, double dt_p) {
+// (TimeEventUpdateNeurons.cpp:78), for plastic networks.  The Poisson devices'
+// clock advances by their own step in a second ring.
+struct TickArgs {
+    double *time_ring;     // [ring]
+    double *time_ring_p;
+    int ring;
+    double dt, dt_p;
+};
+
+__device__ __forceinline__ void tick_body(const TickArgs &a, int32_t k) {
     if (threadIdx.x == 0) {
-        const int32_t k = step.get();
-        time_ring[k % ring] = time_ring[(k - 1) % ring] + dt;
-        time_ring_p[k % ring] = time_ring_p[(k - 1) % ring] + dt_p;
+        a.time_ring[k % a.ring] = a.time_ring[(k - 1) % a.ring] + a.dt;
+        a.time_ring_p[k % a.ring] = a.time_ring_p[(k - 1) % a.ring] + a.dt_p;
     }
+}
+
+// ---------------------------------------------------------------------------
+// The launches around the update kernels, shared by every network of a step.
+// Each of these roles takes 1-3 us of one or a few workgroups, but about
+// 4.6 us as a kernel of its own in a replayed graph, so a step of a circuit
+// spent most of its small kernels on launches.  Roles that do not read each
+// other's results share one:
+//
+// k_step_head, before the updates of step k: the clocks, spike trains and
+// Poisson devices of k and the folds of plastic networks (they read spike
+// lists of updates <= k - 2, weights of update k - 1 and the times of those
+// spikes; the ring has max_delay + 2 slots, so slot k is not among them).
+//
+// k_step_tail, after them: every list of k (populations' and Poisson tiles),
+// the folds of step k + 1 of networks without plastic synapses (they read
+// lists of updates <= k - 1) and, in the first workgroup, the event-queue
+// replay, which reads the tiles.
+//
+// k_step_post, when it has work: post-synaptic learning (reads the lists) and
+// the replay when its sizes do not fit the tail's.
+//
+// The arguments travel by value (pointers read from a table in memory would
+// be flat accesses), so a launch holds a fixed number of roles and a larger
+// circuit takes several.  Per step: two small networks with plastic, train and
+// Poisson inputs (800 AdEx and 200 LIF neurons) 74 us, 91 us with a kernel per
+// role; a 2,501-granule cerebellum 134 and 152 us; 1,000 LIF neurons with
+// Poisson inputs 64 us both ways (one launch less, a longer replay).
+// ---------------------------------------------------------------------------
+constexpr int kHeadRoles = 4, kHeadFolds = 2, kTailLists = 8, kTailFolds = 2, kPostRoles = 8;
+struct FoldRole {
+    FoldTarget target;
+    RingEvents events;
+    int blocks;
+    int lanes;
+};
+struct StepHead {
+    StepRef step;
+    int n_tick, n_train, n_poisson, n_fold;
+    TickArgs tick[kHeadRoles];
+    TrainArgs train[kHeadRoles];
+    int train_blocks[kHeadRoles];
+    PoissonArgs poisson[kHeadRoles];
+    FoldRole fold[kHeadFolds];
+};
+struct StepTail {
+    int n_list, n_fold;
+    CompactArgs list[kTailLists];
+    int list_blocks[kTailLists];
+    FoldRole fold[kTailFolds];
+};
+struct StepPost {
+    int n_post, blocks;     // workgroups per role
+    StdpPostArgs post[kPostRoles];
+};
+
+// kernel arguments are limited to 4 KB
+static_assert(sizeof(StepHead) <= 3584 && sizeof(StepTail) + sizeof(EqArgs) <= 3584 && sizeof(StepPost) <= 3584, "");
+
+__global__ __launch_bounds__(kBlock) void k_step_head(StepHead a) {
+    int b = blockIdx.x;
+    if (b < a.n_tick) {
+        tick_body(a.tick[b], a.step.get());
+        return;
+    }
+    b -= a.n_tick;
+    for (int i = 0; i < a.n_train; i++) {
+        if (b < a.train_blocks[i]) {
+            train_body(a.train[i], b, a.train_blocks[i]);
+            return;
+        }
+        b -= a.train_blocks[i];
+    }
+    for (int i = 0; i < a.n_poisson; i++) {
+        if (b < a.poisson[i].n_tiles) {
+            poisson_body(a.poisson[i], b);
+            return;
+        }
+        b -= a.poisson[i].n_tiles;
+    }
+    for (int i = 0; i < a.n_fold; i++) {
+        if (b < a.fold[i].blocks) {
+            fold_ring_body<0, false>(a.fold[i].target, a.fold[i].events, b, a.fold[i].blocks, a.fold[i].lanes);
+            return;
+        }
+        b -= a.fold[i].blocks;
+    }
+}
+
+// ITEMS: heap entries of the replay in LDS; 0: no replay in this launch.
+template <int ITEMS>
+__global__ __launch_bounds__(kBlock) void k_step_tail(StepTail a, EqArgs q) {
+    int b = blockIdx.x;
+    if (ITEMS > 0) {
+        if (b == 0) {
+            eq_body<ITEMS == 0 ? 1 : ITEMS, kEqFusedDelays>(q);
+            return;
+        }
+        b--;
+    }
+    for (int i = 0; i < a.n_list; i++) {
+        if (b < a.list_blocks[i]) {
+            clock_next_kernel(a.list[i]);
+            compact_body(a.list[i], b, a.list_blocks[i]);
+            return;
+        }
+        b -= a.list_blocks[i];
+    }
+    for (int i = 0; i < a.n_fold; i++) {
+        if (b < a.fold[i].blocks) {
+            if (a.fold[i].events.pulled)
+                fold_ring_body<0, true>(a.fold[i].target, a.fold[i].events, b, a.fold[i].blocks, a.fold[i].lanes);
+            else
+                fold_ring_body<0, false>(a.fold[i].target, a.fold[i].events, b, a.fold[i].blocks, a.fold[i].lanes);
+            return;
+        }
+        b -= a.fold[i].blocks;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void k_step_post(StepPost a) {
+    const int i = (int)blockIdx.x / a.blocks;
+    if (i < a.n_post) stdp_post_body(a.post[i], (int)blockIdx.x % a.blocks, a.blocks);
 }
 
 // Adds every queued event of the population's keys to its conductances, in
