@@ -317,8 +317,10 @@ struct GranuleGroup {
 #pragma unroll
             for (int q = 0; q < 4; q++) in[q] = a.state[(int64_t)(ND + q) * ld + i];
             if (flag) {
-#pragma unroll
-                for (int ty = 0; ty < 3; ty++) in[ty] = fold_key(a, step, ty, i, in[ty]);
+                const bool live[1] = {true};
+                float g[3][1] = {{in[0]}, {in[1]}, {in[2]}};
+                fold_keys<7u, 1>(a, step, i, live, g);
+                for (int ty = 0; ty < 3; ty++) in[ty] = g[ty][0];
             }
             if (EXT) {
                 const uint32_t u = drive_hash_keyed(step_key, i);
