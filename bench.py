@@ -39,7 +39,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK = 8.0e12          # MI355X HBM3E, bytes/s
 BYTES_PER_UPDATE = 32      # V, w, g_exc, g_inh: 16 B read + 16 B written
-BYTES_PER_EVENT = 24       # delivery: 8 B synapse read, 4 B fill atomic, 12 B (order, w) entry
+BYTES_PER_EVENT = 8        # delivery: the 8 B synapse (a densely firing group's targets read all of theirs)
 # VALU issue: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz lane-instructions per second
 VALU_LANE_OPS_PEAK = 256 * 4 * 16 * 2.4e9
 CLOCK_HZ = 2.4e9
