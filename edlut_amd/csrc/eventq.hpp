@@ -527,6 +527,10 @@ __device__ __forceinline__ void eq_window(EqItem *__restrict__ h, const EqArgs &
 
 // The replay of one window by one workgroup of kBlock threads: the spikes
 // per delay are counted by all lanes, the heap operations run on the first wave.
+// Spikes that a wave counts together (others, one by one in the lane that
+// loaded their tile's count).
+constexpr int kEqList = 256;
+
 // LDS_ITEMS heap entries are staged in LDS when the heap cannot outgrow
 // them; MAXD bounds the delays (host-checked).
 template <int LDS_ITEMS, int MAXD>
@@ -539,6 +543,7 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
     __shared__ EqEmitter s_em[kEqMaxEmitters];
     __shared__ int32_t s_scan[kBlock], s_scan2[kBlock];
     __shared__ int32_t s_run, s_base;
+    __shared__ int32_t s_list[kBlock / 64][kEqList];
     __shared__ int32_t s_st[kEqSt];
     __shared__ int32_t s_groups;
     __shared__ double s_delay[MAXD + 1];
@@ -623,11 +628,45 @@ __device__ __forceinline__ void eq_body(const EqArgs &a) {
 #pragma unroll
                 for (int u = 0; u < 8; u++)
                     c8[u] = pre ? pf[u] : eq_g(E.tile_count)[t0 + u * kBlock + (int32_t)threadIdx.x];
+                int32_t mine = 0;
 #pragma unroll
                 for (int u = 0; u < 8; u++) {
-                    const int32_t t = t0 + u * kBlock + (int32_t)threadIdx.x;
-                    if (t >= E.n_tiles) continue;
-                    for (int32_t j = 0; j < c8[u]; j++) count(eq_g(E.staging)[(int64_t)t * E.tile_size + j]);
+                    if (t0 + u * kBlock + (int32_t)threadIdx.x >= E.n_tiles) c8[u] = 0;
+                    mine += c8[u];
+                }
+                // every spike waits for two dependent loads: where a lane has
+                // several, the wave lists their places in the staging rows
+                // and each lane counts one (a step of 800 AdEx and 200 LIF
+                // neurons 61 us, 65 us with each lane counting its own);
+                // with at most one each the list would only add to the wait
+                // (20,011 sparsely firing neurons: 2% when always listed)
+                const bool listed = __ballot(mine > 1) != 0ull;
+                int32_t *const list = s_list[threadIdx.x >> 6];
+                int32_t pos = mine;
+                int32_t total = 0;
+                if (listed) {
+#pragma unroll
+                    for (int off = 1; off < 64; off <<= 1) {
+                        const int32_t v = __shfl_up(pos, off);
+                        pos += eq_lane() >= off ? v : 0;
+                    }
+                    total = __shfl(pos, 63);
+                    pos -= mine;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const int32_t at = (t0 + u * kBlock + (int32_t)threadIdx.x) * E.tile_size;
+                    for (int32_t j = 0; j < c8[u]; j++, pos++) {
+                        if (listed && pos < kEqList) list[pos] = at + j;
+                        else count(eq_g(E.staging)[at + j]);
+                    }
+                }
+                if (listed) {
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    for (int32_t i = eq_lane(); i < total && i < kEqList; i += 64) count(eq_g(E.staging)[list[i]]);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
                 }
             }
         } else {

@@ -53,3 +53,28 @@ def test_heap_depths(oracle, lo, hi, steps, graph):
     assert np.array_equal(st, ost) and np.array_equal(ix, oix)
     for v in range(pop.nv):
         assert np.array_equal(bits(model.GetVectorNeuronState(v)), bits(pop.state(v))), f"variable {v}"
+
+
+@pytest.mark.parametrize("rate", [60.0, 1500.0, 2e4])
+def test_spikes_per_wave(oracle, rate):
+    """Devices of 700 sources with one synapse each (no source has every
+    delay): at most a few spikes in a wave's tiles, some in every tile, and
+    all 700, more than a wave's list holds."""
+    print(f"case spikes per wave rate={rate}", flush=True)
+    n, n_src, hi, steps = 50, 700, 9, 60
+    rng = np.random.default_rng(int(rate))
+    poisson = (np.arange(n_src, dtype=np.int32), rng.integers(0, n, n_src).astype(np.int32),
+               rng.integers(1, hi + 1, n_src).astype(np.int32), np.zeros(n_src, np.uint8),
+               (10.0 ** rng.uniform(-4, -1, n_src)).astype(np.float32))
+    spec = workloads.NetworkSpec("LIFTimeDrivenModel_GPU", "Euler", n, hi, rec=None, steps=steps)
+    spec.poisson.append((workloads.lcg_seeds(31, n_src), rate, poisson))
+    model, net = E.from_spec(spec)
+    pop, onet = oracle.from_spec(spec, LIF_DEFAULTS, np_out_csr)
+    for k, m in ((1, 37), (38, steps - 37)):
+        net.run(m)
+        onet.run(k, m)
+        t_d, _ = net.event_queue()
+        t_o = onet.event_queue()[0]
+        assert np.array_equal(t_d.view(np.uint64), t_o.view(np.uint64))
+    for v in range(pop.nv):
+        assert np.array_equal(bits(model.GetVectorNeuronState(v)), bits(pop.state(v))), f"variable {v}"
