@@ -379,6 +379,8 @@ struct edlut_population {
         t.b_ent = b_ent;
         t.head = head;
         t.node = node;
+        t.n_node = (uint32_t)q_n;
+        t.err = err;
         return t;
     }
 
@@ -1304,8 +1306,9 @@ int err_code(uint32_t e) {
     if (e & 2u)
         return fail(EDLUT_E_CAP, "spike log capacity exceeded (read and clear the log between runs, or raise "
                                  "its capacity)");
-    if (e & 4u) return fail(EDLUT_E_CAP, "input event buffer capacity exceeded");
-    if (e & 8u) return fail(EDLUT_E_STATE, "input fold segment wait exceeded its spin limit");
+    if (e & 4u)
+        return fail(EDLUT_E_STATE, "an update's input events were overwritten: allocation-free updates overlapped on "
+                                   "this GPU");
     if (e & 16u) return fail(EDLUT_E_CAP, "BDF fallback working storage exhausted in one step");
     if (e & 64u) return fail(EDLUT_E_CAP, "event queue capacity exceeded");
     if (e & 128u) return fail(EDLUT_E_STATE, "event queue holds an event of an unknown kind");
@@ -2051,6 +2054,7 @@ int edlut_population_update_noalloc(edlut_population *p, int64_t step, const int
     // 1. ordered fold of the events (position in the arrays = delivery order)
     FoldTarget t = p->fold_target((int)(++p->upd_seq & 1u));
     t.node = (FoldNode *)base;
+    t.n_node = (uint32_t)n_events;
     launch_push_fold(t, PushEvents{target, type, weight, n_events, (int32_t)p->n, p->mask & 7u, p->err}, st);
     // 2. integrate, detect, compact into the caller's spike list
     UpdateArgs a = make_update_args(p, (int32_t)step);

@@ -9,6 +9,7 @@
 #include <type_traits>
 #include "device_common.hpp"
 #include "device_models.hpp"
+#include "event_list.hpp"
 #include "eventq.hpp"
 
 namespace edl {
@@ -50,13 +51,6 @@ struct FoldEntry {
     uint32_t pad;
 };
 
-// One host-pushed event: its weight and the event that reached the key's list
-// before it (1 + its number; 0 ends the list).
-struct FoldNode {
-    uint32_t next;
-    float w;
-};
-
 struct FoldTarget {
     float *state;
     int64_t stride;
@@ -68,6 +62,8 @@ struct FoldTarget {
     FoldEntry *b_ent;    // network mode: event buffer (order key, weight)
     uint32_t *head;      // plug-in mode, per key: 1 + its last listed event (0: none)
     FoldNode *node;      // plug-in mode: the step's events
+    uint32_t n_node;     // their number
+    uint32_t *err;       // bit 2: a list of events was overwritten
     // network mode: fixed segment of each key (prefix of the keys' synapse
     // counts; a synapse carries at most one event per step), null otherwise
     const uint64_t *seg_off;
@@ -248,38 +244,10 @@ __device__ __attribute__((noinline)) float fold_sorted(FoldEntry *ent, const Ran
 }
 
 // Plug-in mode: adds the events listed from `hd` to g in the order of their
-// numbers and clears the list.  Each walk finds the next four of them, so a
-// list of up to four takes two walks.
-__device__ __attribute__((noinline)) float fold_list(uint32_t *head, const FoldNode *node, uint64_t key, uint32_t hd,
-                                                     float g) {
-    uint32_t last = 0u;
-    const FoldNode first = node[hd - 1u];
-    if (first.next == 0u) {
-        g = g + first.w;
-    } else {
-        for (;;) {
-            uint32_t b0 = ~0u, b1 = ~0u, b2 = ~0u, b3 = ~0u;
-            float w0 = 0.0f, w1 = 0.0f, w2 = 0.0f, w3 = 0.0f;
-            for (uint32_t q = hd; q != 0u;) {
-                const FoldNode e = node[q - 1u];
-                if (q > last && q < b3) {
-                    b3 = q;
-                    w3 = e.w;
-                    if (b3 < b2) { const uint32_t t = b2; b2 = b3; b3 = t; const float u = w2; w2 = w3; w3 = u; }
-                    if (b2 < b1) { const uint32_t t = b1; b1 = b2; b2 = t; const float u = w1; w1 = w2; w2 = u; }
-                    if (b1 < b0) { const uint32_t t = b0; b0 = b1; b1 = t; const float u = w0; w0 = w1; w1 = u; }
-                }
-                q = e.next;
-            }
-            if (b0 == ~0u) break;
-            g = g + w0;
-            if (b1 != ~0u) g = g + w1;
-            if (b2 != ~0u) g = g + w2;
-            if (b3 == ~0u) break;
-            g = g + w3;
-            last = b3;
-        }
-    }
+// numbers and clears the list.
+__device__ __attribute__((noinline)) float fold_list(uint32_t *head, FoldNode *node, uint32_t n_node, uint32_t *err,
+                                                     uint64_t key, uint32_t hd, float g) {
+    if (!event_list_add(eq_g(node), n_node, hd, g)) atomicOr(err, 4u);
     head[key] = 0u;
     return g;
 }
@@ -390,7 +358,7 @@ __device__ __forceinline__ void fold_keys(const UpdateArgs &a, int32_t step, uin
                 if (!((MASK >> ty) & 1u) || !live[n]) continue;
                 const uint64_t key = (uint64_t)ty * (uint64_t)a.stride + (uint64_t)(i0 + n * kWave);
                 const uint32_t hd = t.head[key];
-                if (hd) g[ty][n] = fold_list(t.head, t.node, key, hd, g[ty][n]);
+                if (hd) g[ty][n] = fold_list(t.head, t.node, t.n_node, t.err, key, hd, g[ty][n]);
             }
         return;
     }

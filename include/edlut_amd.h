@@ -154,7 +154,10 @@ int edlut_population_get_spikes(const edlut_population *pop, int32_t *idx, int c
  * is a library-wide device array of EDLUT_NOALLOC_MAX_EVENTS events (8 MiB,
  * held by each GPU the library runs on until the process ends): n_events
  * above it is refused (EDLUT_E_CAP).  Every call on one GPU shares that
- * array, so calls that overlap on one GPU race; serialise them.  An event
+ * array, so calls that overlap on one GPU race: serialise them.  Updates that
+ * overlapped use wrong or missing events; where one finds its list of events
+ * overwritten the population's next synchronous call reports it
+ * (EDLUT_E_STATE).  An event
  * whose target is out of range or whose synapse type is not enabled is
  * dropped and reported (EDLUT_E_ARG) by the population's next synchronous
  * call.  Refused while events queued by edlut_population_push_inputs wait.

@@ -1,0 +1,143 @@
+"""The plug-in fold's list of one key's events (csrc/event_list.hpp), compiled
+for the host: sums in the order of the events' numbers whatever the order of
+arrival, and an end within the list's nodes on any contents, as when the nodes
+of an allocation-free update are overwritten by a call that overlaps it.
+"""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PROGRAM = r"""
+#define __host__
+#define __device__
+#include "event_list.hpp"
+#include <algorithm>
+#include <cmath>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <random>
+#include <vector>
+using edl::FoldNode;
+
+// n nodes, every access checked and counted; past `budget` accesses the
+// program ends.
+struct Checked {
+    std::vector<FoldNode> *v;
+    long *used;
+    long budget;
+    FoldNode &operator[](uint32_t i) const {
+        if (i >= v->size()) { std::printf("node %u of %zu\n", i, v->size()); std::exit(2); }
+        if (++*used > budget) { std::printf("%ld accesses\n", *used); std::exit(3); }
+        return (*v)[i];
+    }
+};
+
+static std::mt19937 rng(7);
+static uint32_t below(uint32_t n) { return rng() % n; }
+
+// Events 1..n, every `every`-th on the key, in blocks of `block` that arrive
+// in random order, each block in ascending or descending order.
+static std::vector<uint32_t> arrivals(uint32_t n, uint32_t every, uint32_t block, bool ascending) {
+    std::vector<std::vector<uint32_t>> b;
+    for (uint32_t q = 1; q <= n; q += every) {
+        if (b.empty() || b.back().size() == block) b.emplace_back();
+        b.back().push_back(q);
+    }
+    std::shuffle(b.begin(), b.end(), rng);
+    std::vector<uint32_t> out;
+    for (auto &x : b) {
+        if (!ascending) std::reverse(x.begin(), x.end());
+        out.insert(out.end(), x.begin(), x.end());
+    }
+    return out;
+}
+
+static uint32_t build(std::vector<FoldNode> &v, const std::vector<uint32_t> &order) {
+    uint32_t hd = 0;
+    for (uint32_t q : order) {
+        v[q - 1].next = hd;
+        hd = q;
+    }
+    return hd;
+}
+
+static void fill(std::vector<FoldNode> &v) {
+    for (auto &x : v) x = FoldNode{0xdeadbeefu, std::pow(10.0f, (float)below(800) / 100.0f - 6.0f)};
+}
+
+static int sums(long per_node) {
+    for (uint32_t m : {1u, 2u, 3u, 4u, 5u, 8u, 9u, 15u, 16u, 17u, 18u, 33u, 64u, 65u, 200u, 1000u, 5000u})
+        for (uint32_t every : {1u, 3u})
+            for (uint32_t block : {1u, 7u, 64u, 100000u})
+                for (bool asc : {false, true}) {
+                    const uint32_t n = (m - 1) * every + 1;
+                    std::vector<FoldNode> v(n);
+                    fill(v);
+                    float want = 0.25f, got = 0.25f;
+                    for (uint32_t q = 1; q <= n; q += every) want = want + v[q - 1].w;
+                    const uint32_t hd = build(v, arrivals(n, every, block, asc));
+                    long used = 0;
+                    const long budget = per_node > 0 ? per_node * m : (long)m * m + 64;
+                    if (!edl::event_list_add(Checked{&v, &used, budget}, n, hd, got) ||
+                        std::memcmp(&got, &want, 4)) {
+                        std::printf("m %u every %u block %u asc %d: %.9g, not %.9g\n", m, every, block, asc, got, want);
+                        return 1;
+                    }
+                }
+    return 0;
+}
+
+// Lists with some of their nodes overwritten by another list of the same or
+// another number of events, or by anything.
+static int overwritten(long per_node) {
+    int refused = 0;
+    for (int t = 0; t < 20000; t++) {
+        const uint32_t n = 1 + below(t % 7 == 0 ? 3000 : 40);
+        std::vector<FoldNode> v(n);
+        fill(v);
+        const uint32_t hd = build(v, arrivals(n, 1 + below(3), 1 + below(80), below(2)));
+        for (uint32_t k = 0; k <= below(6); k++) {
+            const uint32_t at = below(n);
+            const uint32_t what = below(6);
+            v[at].next = what == 0 ? at + 1 : what == 1 ? hd : what == 2 ? below(2 * n) : what == 3 ? ~0u : 1 + below(n);
+        }
+        float g = 0.0f;
+        long used = 0;
+        const long budget = per_node > 0 ? per_node * n : (long)n * n + 64;
+        refused += !edl::event_list_add(Checked{&v, &used, budget}, n, hd, g);
+    }
+    return refused > 1000 ? 0 : 1;
+}
+
+int main(int argc, char **argv) {
+    const long per_node = std::atol(argv[2]);
+    return std::strcmp(argv[1], "sums") ? overwritten(per_node) : sums(per_node);
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def program(tmp_path_factory):
+    d = tmp_path_factory.mktemp("event_list")
+    src, exe = d / "check.cpp", d / "check"
+    src.write_text(PROGRAM)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-ffp-contract=off", "-I",
+                    os.path.join(ROOT, "edlut_amd", "csrc"), "-o", str(exe), str(src)], check=True)
+    return str(exe)
+
+
+def _run(*args):
+    r = subprocess.run(args, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, (r.returncode, r.stdout, r.stderr)
+
+
+def test_sums_in_order(program):
+    _run(program, "sums", "0")
+
+
+def test_overwritten_lists_end(program):
+    _run(program, "overwritten", "0")
