@@ -7,45 +7,141 @@ namespace edl {
 
 // One host-pushed event: its weight and the event that reached the key's list
 // before it (1 + its number; 0 ends the list).
-struct FoldNode {
+struct alignas(8) FoldNode {
     uint32_t next;
     float w;
 };
 
+// Lists of up to this many events are summed by selection, longer ones sorted
+// first.  An update of one AdEx cell, of 8 and of 64 cells with 96 events on
+// each takes 237, 736 and 508 us by selection, with 97 (sorted) 174, 727 and
+// 513 us.
+constexpr uint32_t kListShort = 96;
+
+// Sorts the list from `hd` by event number: its runs (a wave's events arrive
+// together, in descending order seen from the head) are merged two by two
+// through `next`, pass by pass.  Returns the new head, 0 when the chain is no
+// list of at most n nodes numbered 1 to n.
+template <class Nodes>
+__host__ __device__ inline uint32_t event_list_sort(Nodes node, uint32_t n, uint32_t hd) {
+    uint32_t m = 0u, prev = 0u;
+    for (uint32_t q = hd; q != 0u; m++) {
+        if (q > n || m == n) return 0u;
+        const uint32_t next = node[q - 1u].next;
+        node[q - 1u].next = prev;
+        prev = q;
+        q = next;
+    }
+    hd = prev;
+    // a pass at least halves the runs
+    for (int pass = 0; pass < 32; pass++) {
+        uint32_t runs = 0u, left = m, ahead = m, tail = 0u, p = hd;
+        while (p != 0u) {
+            // x: the run from p to e; y: the one after it
+            uint32_t x = p, e = p, y;
+            for (;;) {
+                y = node[e - 1u].next;
+                if (y > n || ahead-- == 0u) return 0u;
+                if (y <= e) break;
+                e = y;
+            }
+            bool more_x = true, more_y = y != 0u;
+            p = 0u;
+            runs++;
+            if (!more_y && tail == 0u) return hd;   // one run: sorted
+            while (more_x || more_y) {
+                const bool take_x = more_x && (!more_y || x < y);
+                const uint32_t t = take_x ? x : y;
+                const uint32_t next = node[t - 1u].next;
+                if (next > n || left-- == 0u) return 0u;
+                if (tail != 0u) node[tail - 1u].next = t;
+                else hd = t;
+                tail = t;
+                if (take_x) {
+                    more_x = t != e;
+                    x = next;
+                    if (more_x && x == 0u) return 0u;
+                } else {
+                    more_y = next > t;
+                    if (more_y) y = next;
+                    else p = next;
+                }
+            }
+        }
+        node[tail - 1u].next = 0u;
+        if (runs == 1u) return hd;
+    }
+    return 0u;
+}
+
 // Adds the events listed from `hd` (not 0) to g in the order of their numbers.
-// Each walk finds the next four of them, so a list of up to four takes one.
+// The loads along the chain bound it: each waits for the one before.  A walk
+// finds the next four events, so a list of up to four takes one and one of m
+// events m / 4.  A long list is sorted first, which takes a walk to turn it
+// round and about one and a half for each doubling of its runs: an update of one
+// cell with 1,000 events 3.4 ms, with 3,000 12.6 ms (by selection 19.2 and
+// 170 ms), with 100,000 0.65 s.
 // False when the chain is no list of at most n nodes numbered 1 to n: the
 // allocation-free updates of one GPU share their nodes, and a call that
 // overlaps another overwrites its lists.  Every loop ends on any contents, and
 // no access leaves the n nodes.
 template <class Nodes>
 __host__ __device__ inline bool event_list_add(Nodes node, uint32_t n, uint32_t hd, float &g) {
-    uint32_t last = 0u;
-    for (uint32_t done = 4u;; done += 4u) {
-        uint32_t b0 = ~0u, b1 = ~0u, b2 = ~0u, b3 = ~0u, m = 0u;
-        float w0 = 0.0f, w1 = 0.0f, w2 = 0.0f, w3 = 0.0f;
-        for (uint32_t q = hd; q != 0u; m++) {
-            if (q > n || m == n) return false;
-            const uint32_t next = node[q - 1u].next;
-            const float w = node[q - 1u].w;
-            if (q > last && q < b3) {
-                b3 = q;
-                w3 = w;
-                if (b3 < b2) { const uint32_t t = b2; b2 = b3; b3 = t; const float u = w2; w2 = w3; w3 = u; }
-                if (b2 < b1) { const uint32_t t = b1; b1 = b2; b2 = t; const float u = w1; w1 = w2; w2 = u; }
-                if (b1 < b0) { const uint32_t t = b0; b0 = b1; b1 = t; const float u = w0; w0 = w1; w1 = u; }
-            }
-            q = next;
+    uint32_t last = 0u, b0, b1, b2, b3, q, m = 0u;
+    float w0, w1, w2, w3;
+    auto none = [&]() {
+        b0 = b1 = b2 = b3 = ~0u;
+        w0 = w1 = w2 = w3 = 0.0f;
+    };
+    // event q to the first four after `last`
+    auto pick = [&](uint32_t q, float w) {
+        if (q > last && q < b3) {
+            b3 = q;
+            w3 = w;
+            if (b3 < b2) { const uint32_t t = b2; b2 = b3; b3 = t; const float u = w2; w2 = w3; w3 = u; }
+            if (b2 < b1) { const uint32_t t = b1; b1 = b2; b2 = t; const float u = w1; w1 = w2; w2 = u; }
+            if (b1 < b0) { const uint32_t t = b0; b0 = b1; b1 = t; const float u = w0; w0 = w1; w1 = u; }
         }
-        if (b0 == ~0u) return false;
-        g = g + w0;
-        if (b1 != ~0u) g = g + w1;
-        if (b2 != ~0u) g = g + w2;
-        if (b3 != ~0u) g = g + w3;
-        if (m <= done) return true;
-        if (b3 == ~0u) return false;
-        last = b3;
+    };
+    none();
+    // (0, the end of the list, is past n as well)
+    for (q = hd; (q - 1u < n) & (m < kListShort); m++) {
+        const uint32_t at = q - 1u;
+        const uint32_t next = node[at].next;
+        const float w = node[at].w;
+        pick(q, w);
+        q = next;
     }
+    if (q == 0u) {
+        // one walk for every four events; the first one knows their number
+        for (uint32_t done = 0u;;) {
+            g = g + w0;
+            if (b1 != ~0u) g = g + w1;
+            if (b2 != ~0u) g = g + w2;
+            if (b3 != ~0u) g = g + w3;
+            done += 4u;
+            if (done >= m) return b0 != ~0u;
+            if (b3 == ~0u) return false;
+            last = b3;
+            none();
+            q = hd;
+            for (uint32_t i = 0; i < m; i++) {
+                const uint32_t at = q - 1u < n ? q - 1u : n - 1u;
+                const uint32_t next = node[at].next;
+                const float w = node[at].w;
+                pick(q, w);
+                q = next;
+            }
+        }
+    }
+    q = q <= n ? event_list_sort(node, n, hd) : 0u;
+    if (q == 0u) return false;
+    for (uint32_t left = n; q != 0u; left--) {
+        if (q > n || left == 0u) return false;
+        g = g + node[q - 1u].w;
+        q = node[q - 1u].next;
+    }
+    return true;
 }
 
 }  // namespace edl

@@ -70,7 +70,7 @@ static void fill(std::vector<FoldNode> &v) {
 }
 
 static int sums(long per_node) {
-    for (uint32_t m : {1u, 2u, 3u, 4u, 5u, 8u, 9u, 15u, 16u, 17u, 18u, 33u, 64u, 65u, 200u, 1000u, 5000u})
+    for (uint32_t m : {1u, 2u, 3u, 4u, 5u, 8u, 9u, 15u, 16u, 17u, 33u, 64u, 65u, 95u, 96u, 97u, 98u, 200u, 1000u, 5000u})
         for (uint32_t every : {1u, 3u})
             for (uint32_t block : {1u, 7u, 64u, 100000u})
                 for (bool asc : {false, true}) {
@@ -136,8 +136,8 @@ def _run(*args):
 
 
 def test_sums_in_order(program):
-    _run(program, "sums", "0")
+    _run(program, "sums", "60")
 
 
 def test_overwritten_lists_end(program):
-    _run(program, "overwritten", "0")
+    _run(program, "overwritten", "240")

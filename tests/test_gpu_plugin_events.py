@@ -41,7 +41,7 @@ def _state(m, o):
         assert np.array_equal(bits(m.GetVectorNeuronState(v)), bits(o.state(v).astype(np.float32))), f"var {v}"
 
 
-@pytest.mark.parametrize("per_key", [1, 2, 3, 4, 5, 8, 9, 33, 200])
+@pytest.mark.parametrize("per_key", [1, 2, 3, 4, 5, 8, 9, 33, 96, 97, 200, 5000])
 def test_events_of_one_key(oracle, per_key):
     """Weights over eight decades make every order of the sum visible."""
     print(f"case events of one key {per_key}", flush=True)
