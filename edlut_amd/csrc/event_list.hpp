@@ -77,71 +77,66 @@ __host__ __device__ inline uint32_t event_list_sort(Nodes node, uint32_t n, uint
 // Adds the events listed from `hd` (not 0) to g in the order of their numbers.
 // The loads along the chain bound it: each waits for the one before.  A walk
 // finds the next four events, so a list of up to four takes one and one of m
-// events m / 4.  A long list is sorted first, which takes a walk to turn it
-// round and about one and a half for each doubling of its runs: an update of one
-// cell with 1,000 events 3.4 ms, with 3,000 12.6 ms (by selection 19.2 and
-// 170 ms), with 100,000 0.65 s.
-// False when the chain is no list of at most n nodes numbered 1 to n: the
-// allocation-free updates of one GPU share their nodes, and a call that
-// overlaps another overwrites its lists.  Every loop ends on any contents, and
-// no access leaves the n nodes.
+// events m / 4.
+// kListLong: more than kListShort events, nothing added.  kListBad: the chain is
+// no list of at most n nodes numbered 1 to n (the allocation-free updates of
+// one GPU share their nodes, and a call that overlaps another overwrites its
+// lists).  Every loop ends on any contents, and no access leaves the n nodes.
+enum ListEnd : uint32_t { kListDone = 0, kListLong = 1, kListBad = 2 };
 template <class Nodes>
-__host__ __device__ inline bool event_list_add(Nodes node, uint32_t n, uint32_t hd, float &g) {
-    uint32_t last = 0u, b0, b1, b2, b3, q, m = 0u;
-    float w0, w1, w2, w3;
-    auto none = [&]() {
-        b0 = b1 = b2 = b3 = ~0u;
-        w0 = w1 = w2 = w3 = 0.0f;
-    };
-    // event q to the first four after `last`
-    auto pick = [&](uint32_t q, float w) {
-        if (q > last && q < b3) {
-            b3 = q;
-            w3 = w;
-            if (b3 < b2) { const uint32_t t = b2; b2 = b3; b3 = t; const float u = w2; w2 = w3; w3 = u; }
-            if (b2 < b1) { const uint32_t t = b1; b1 = b2; b2 = t; const float u = w1; w1 = w2; w2 = u; }
-            if (b1 < b0) { const uint32_t t = b0; b0 = b1; b1 = t; const float u = w0; w0 = w1; w1 = u; }
-        }
-    };
-    none();
-    // (0, the end of the list, is past n as well)
-    for (q = hd; (q - 1u < n) & (m < kListShort); m++) {
-        const uint32_t at = q - 1u;
-        const uint32_t next = node[at].next;
-        const float w = node[at].w;
-        pick(q, w);
-        q = next;
+__host__ __device__ inline ListEnd event_list_add(Nodes node, uint32_t n, uint32_t hd, float &g) {
+    if (hd > n) return kListBad;
+    const uint32_t next1 = node[hd - 1u].next;
+    const float first = node[hd - 1u].w;
+    if (next1 == 0u) {
+        g = g + first;
+        return kListDone;
     }
-    if (q == 0u) {
-        // one walk for every four events; the first one knows their number
-        for (uint32_t done = 0u;;) {
-            g = g + w0;
-            if (b1 != ~0u) g = g + w1;
-            if (b2 != ~0u) g = g + w2;
-            if (b3 != ~0u) g = g + w3;
-            done += 4u;
-            if (done >= m) return b0 != ~0u;
-            if (b3 == ~0u) return false;
-            last = b3;
-            none();
-            q = hd;
-            for (uint32_t i = 0; i < m; i++) {
-                const uint32_t at = q - 1u < n ? q - 1u : n - 1u;
-                const uint32_t next = node[at].next;
-                const float w = node[at].w;
-                pick(q, w);
-                q = next;
+    uint32_t last = 0u, q, m = 0u;
+    for (uint32_t done = 4u;; done += 4u) {
+        uint32_t b0 = ~0u, b1 = ~0u, b2 = ~0u, b3 = ~0u, i = 0u;
+        float w0 = 0.0f, w1 = 0.0f, w2 = 0.0f, w3 = 0.0f;
+        // the first walk counts the events (0, the end, is past n as well), the
+        // others keep to their number
+        const uint32_t limit = m == 0u ? kListShort : m;
+        for (q = hd; (q - 1u < n) & (i < limit); i++) {
+            const uint32_t next = node[q - 1u].next;
+            const float w = node[q - 1u].w;
+            if (q > last && q < b3) {
+                b3 = q;
+                w3 = w;
+                if (b3 < b2) { const uint32_t t = b2; b2 = b3; b3 = t; const float u = w2; w2 = w3; w3 = u; }
+                if (b2 < b1) { const uint32_t t = b1; b1 = b2; b2 = t; const float u = w1; w1 = w2; w2 = u; }
+                if (b1 < b0) { const uint32_t t = b0; b0 = b1; b1 = t; const float u = w0; w0 = w1; w1 = u; }
             }
+            q = next;
         }
+        if (q != 0u) return m == 0u && q <= n ? kListLong : kListBad;
+        m = i;
+        g = g + w0;
+        if (b1 != ~0u) g = g + w1;
+        if (b2 != ~0u) g = g + w2;
+        if (b3 != ~0u) g = g + w3;
+        if (done >= m) return b0 != ~0u ? kListDone : kListBad;
+        if (b3 == ~0u) return kListBad;
+        last = b3;
     }
-    q = q <= n ? event_list_sort(node, n, hd) : 0u;
-    if (q == 0u) return false;
+}
+
+// The same for a list that is longer: sorted, which takes a walk to turn it
+// round and about one and a half for each doubling of its runs, and added in one.
+// An update of one cell with 1,000 events 3.4 ms, with 3,000 12.6 ms (by
+// selection 19.2 and 170 ms), with 100,000 0.65 s.
+template <class Nodes>
+__host__ __device__ inline ListEnd event_list_add_long(Nodes node, uint32_t n, uint32_t hd, float &g) {
+    uint32_t q = event_list_sort(node, n, hd);
+    if (q == 0u) return kListBad;
     for (uint32_t left = n; q != 0u; left--) {
-        if (q > n || left == 0u) return false;
+        if (q > n || left == 0u) return kListBad;
         g = g + node[q - 1u].w;
         q = node[q - 1u].next;
     }
-    return true;
+    return kListDone;
 }
 
 }  // namespace edl

@@ -244,12 +244,18 @@ __device__ __attribute__((noinline)) float fold_sorted(FoldEntry *ent, const Ran
 }
 
 // Plug-in mode: adds the events listed from `hd` to g in the order of their
-// numbers and clears the list.
-__device__ __attribute__((noinline)) float fold_list(uint32_t *head, FoldNode *node, uint32_t n_node, uint32_t *err,
-                                                     uint64_t key, uint32_t hd, float g) {
-    if (!event_list_add(eq_g(node), n_node, hd, g)) atomicOr(err, 4u);
-    head[key] = 0u;
-    return g;
+// numbers, or leaves a long list for fold_list_long.
+struct FoldSum {
+    float g;
+    uint32_t end;   // ListEnd
+};
+__device__ __attribute__((noinline)) FoldSum fold_list(FoldNode *node, uint32_t n_node, uint32_t hd, float g) {
+    const uint32_t end = event_list_add(eq_g(node), n_node, hd, g);
+    return FoldSum{g, end};
+}
+__device__ __attribute__((noinline)) FoldSum fold_list_long(FoldNode *node, uint32_t n_node, uint32_t hd, float g) {
+    const uint32_t end = event_list_add_long(eq_g(node), n_node, hd, g);
+    return FoldSum{g, end};
 }
 
 struct ExtDrive {
@@ -351,6 +357,7 @@ __device__ __forceinline__ void fold_keys(const UpdateArgs &a, int32_t step, uin
                                           float (&g)[3][ITEMS]) {
     const FoldTarget &t = a.fold;
     if (!t.seg_off) {
+        uint32_t more = 0u, bad = 0u;   // keys of long lists, by ty * ITEMS + n
 #pragma unroll
         for (int n = 0; n < ITEMS; n++)
 #pragma unroll
@@ -358,8 +365,27 @@ __device__ __forceinline__ void fold_keys(const UpdateArgs &a, int32_t step, uin
                 if (!((MASK >> ty) & 1u) || !live[n]) continue;
                 const uint64_t key = (uint64_t)ty * (uint64_t)a.stride + (uint64_t)(i0 + n * kWave);
                 const uint32_t hd = t.head[key];
-                if (hd) g[ty][n] = fold_list(t.head, t.node, t.n_node, t.err, key, hd, g[ty][n]);
+                if (!hd) continue;
+                const FoldSum s = fold_list(t.node, t.n_node, hd, g[ty][n]);
+                g[ty][n] = s.g;
+                bad |= s.end & kListBad;
+                if (s.end == kListLong) more |= 1u << (ty * ITEMS + n);
+                else t.head[key] = 0u;
             }
+        while (more) {
+            const int x = __builtin_ctz(more);
+            more &= more - 1u;
+            const uint64_t key = (uint64_t)(x / ITEMS) * (uint64_t)a.stride + (uint64_t)(i0 + (x % ITEMS) * kWave);
+            float gx = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 3 * ITEMS; q++) gx = x == q ? g[q / ITEMS][q % ITEMS] : gx;
+            const FoldSum s = fold_list_long(t.node, t.n_node, t.head[key], gx);
+            bad |= s.end & kListBad;
+            t.head[key] = 0u;
+#pragma unroll
+            for (int q = 0; q < 3 * ITEMS; q++) g[q / ITEMS][q % ITEMS] = x == q ? s.g : g[q / ITEMS][q % ITEMS];
+        }
+        if (bad) atomicOr(t.err, 4u);
         return;
     }
     uint32_t m[3][ITEMS];
