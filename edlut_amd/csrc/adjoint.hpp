@@ -17,7 +17,10 @@
 // steps into LDS.  The adjoint recurrence is linear in the adjoint state, so
 // the backward pass runs every checkpoint segment at once:
 //
-//   k_fit_forward  V trace [steps][n]; state + event cursor every `seg` steps
+//   k_fit_forward  V trace [steps][n]; state + event cursor every `keep`
+//                  segments of `seg` steps
+//   k_fit_expand   (keep > 1) per (kept checkpoint, neuron): the forward pass
+//                  again from there, giving every segment's state and cursor
 //   k_fit_maps     per (segment, neuron): the affine map from the adjoint
 //                  state at the segment's end to the one at its start
 //   k_fit_scan     per neuron: those maps applied from the last segment to
@@ -65,10 +68,14 @@ struct FitArgs {
     uint8_t *spikes;                             // [steps][n] (optional)
     float *traj;                                 // [steps][4][n] state before integration (optional)
     int32_t *traj_since;                         // [steps][n] refractory count (optional)
-    float *ck_state;                             // [segs][4][n]
-    int32_t *ck_int;                             // [segs+1][2][n]: event cursor, last spike
+    int keep;                                    // segments per checkpoint
+    float *kept_state;                           // [checkpoints+1][4][n]
+    int32_t *kept_int;                           // [checkpoints+1][2][n]: event cursor, last spike
     // backward: segments [c_lo, c_hi) of this launch
     int c_lo, c_hi;
+    int ck_lo;                                   // segment of the first row below
+    float *ck_state;                             // [segments][4][n]
+    int32_t *ck_int;                             // [segments+1][2][n]: event cursor, last spike
     const float *grad_v;                         // [steps][n]
     float *grad_par;                             // [4][n]: g_leak e_leak tau_exc tau_inh
     float *grad_w;                               // [n][n_syn]
@@ -211,7 +218,9 @@ struct FitEvents {
 // are 0: adding it changes nothing), and a bit for the steps that have more,
 // whose events wave 0 then walks itself.  Lanes past the last neuron repeat
 // it (the same values to the same places).  EXTRA: with the optional outputs,
-// or with a refractory table too long for LDS.
+// with a refractory table too long for LDS, or with checkpoints further apart
+// than segments (the counters of their rows in the other variants take the LIF
+// forward of 256 neurons from 1.64 to 1.75 ms).
 //
 // 256 neurons, 10,000 steps: 1.63 ms (LIF) and 4.7 ms (AdEx).  With the events
 // walked inside the recurrence (three dependent loads in nearly every step of
@@ -295,21 +304,27 @@ __global__ __launch_bounds__(2 * kFitBlock) void k_fit_forward(FitArgs a) {
     int since = a.refr_len;
     const float frac0 = refr_lds ? s_refr[0] : 1.0f;
     float *vt = a.v_trace + i;
+    int row = 0, to_keep = 1;   // checkpoint row, segments it still takes
     for (int c = 0; c < a.segs; c++) {
         const int buf = c & 1;
         if (producer) {
             if (c + 1 < a.segs) fill(c + 1, buf ^ 1);
-            else a.ck_int[(int64_t)a.segs * 2 * a.n + i] = e;   // cursor past the last event
+            else a.kept_int[(int64_t)(EXTRA ? (a.segs + a.keep - 1) / a.keep : a.segs) * 2 * a.n + i] = e;   // past the last event
         } else {
             const int k0 = c * a.seg + 1, k1 = min(a.steps, (c + 1) * a.seg);
-            float *cs = a.ck_state + (int64_t)c * 4 * a.n;
+            // a row is written over until its last segment, the kept one
+            float *cs = a.kept_state + (int64_t)(EXTRA ? row : c) * 4 * a.n;
             cs[i] = V;
             cs[a.n + i] = W;
             cs[2 * a.n + i] = ge;
             cs[3 * a.n + i] = gi;
-            int32_t *ci = a.ck_int + (int64_t)c * 2 * a.n;
+            int32_t *ci = a.kept_int + (int64_t)(EXTRA ? row : c) * 2 * a.n;
             ci[i] = s_cur[buf][lane];
             ci[a.n + i] = last;
+            if (EXTRA && --to_keep == 0) {
+                to_keep = a.keep;
+                row++;
+            }
             int cur = s_cur[buf][lane];   // events up to it belong to earlier steps
             uint32_t any = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_any[buf]);
             const float *in = &s_in[buf][0][0][lane];
@@ -382,9 +397,9 @@ template <int MODEL>
 __device__ __forceinline__ void fit_replay(const FitArgs &a, int c, int i, float gl, float el, float cfe,
                                            float cfi, float (*s)[kFitSeg][kFitBlock]) {
     const int lane = (int)threadIdx.x;
-    const float *cs = a.ck_state + (int64_t)c * 4 * a.n;
+    const float *cs = a.ck_state + (int64_t)(c - a.ck_lo) * 4 * a.n;
     float V = cs[i], W = cs[a.n + i], ge = cs[2 * a.n + i], gi = cs[3 * a.n + i];
-    const int32_t *ci = a.ck_int + (int64_t)c * 2 * a.n;
+    const int32_t *ci = a.ck_int + (int64_t)(c - a.ck_lo) * 2 * a.n;
     int last = ci[a.n + i];
     FitEvents ev;
     ev.seek(a, i, ci[i]);
@@ -405,6 +420,43 @@ __device__ __forceinline__ void fit_replay(const FitArgs &a, int c, int i, float
             fit_step<MODEL>(a, gl, el, cfe, cfi, 1.0f, V, W, ge, gi);
         }
     }
+}
+
+// Segments c_lo to c_hi from their kept checkpoints (c_lo is one), one lane
+// per (checkpoint, neuron): the forward pass again, its state and event cursor
+// written at every segment's start, the cursor also past the last one.
+template <int MODEL>
+__global__ __launch_bounds__(kFitBlock) void k_fit_expand(FitArgs a) {
+    const int64_t q = (int64_t)blockIdx.x * kFitBlock + threadIdx.x;
+    const int i = (int)(q % a.n);
+    const int64_t c0 = a.c_lo + q / a.n * a.keep;
+    if (c0 >= a.c_hi) return;
+    const int c1 = (int)min(c0 + a.keep, (int64_t)a.c_hi);
+    const float gl = a.gl[i], el = a.el[i];
+    const float cfe = expf(-a.h / a.te[i]), cfi = expf(-a.h / a.ti[i]);
+    const float *ks = a.kept_state + c0 / a.keep * 4 * a.n;
+    float V = ks[i], W = ks[a.n + i], ge = ks[2 * a.n + i], gi = ks[3 * a.n + i];
+    const int32_t *ki = a.kept_int + c0 / a.keep * 2 * a.n;
+    int last = ki[a.n + i];
+    FitEvents ev;
+    ev.seek(a, i, ki[i]);
+    for (int c = (int)c0; c < c1; c++) {
+        float *cs = a.ck_state + (int64_t)(c - a.ck_lo) * 4 * a.n;
+        cs[i] = V;
+        cs[a.n + i] = W;
+        cs[2 * a.n + i] = ge;
+        cs[3 * a.n + i] = gi;
+        int32_t *ci = a.ck_int + (int64_t)(c - a.ck_lo) * 2 * a.n;
+        ci[i] = ev.e;
+        ci[a.n + i] = last;
+        const int k1 = min(a.steps, (c + 1) * a.seg);
+        for (int k = c * a.seg + 1; k <= k1; k++) {
+            ev.apply(k, ge, gi);
+            const float frac = MODEL == 0 ? lif_frac(a, k - 1 - last) : 1.0f;
+            if (fit_step<MODEL>(a, gl, el, cfe, cfi, frac, V, W, ge, gi)) last = k;
+        }
+    }
+    if (c1 == a.c_hi) a.ck_int[(int64_t)(c1 - a.ck_lo) * 2 * a.n + i] = ev.e;
 }
 
 // The vector-Jacobian product of one AdEx step (without its reset): (lV, lW,
@@ -670,7 +722,8 @@ __global__ __launch_bounds__(kFitGradBlock) void k_fit_grads(FitArgs a) {
             a.carry[(int64_t)(4 + tid) * a.n + i] = x;
         }
     }
-    const int e_lo = a.ck_int[(int64_t)a.c_lo * 2 * a.n + i], e_hi = a.ck_int[(int64_t)a.c_hi * 2 * a.n + i];
+    const int e_lo = a.ck_int[(int64_t)(a.c_lo - a.ck_lo) * 2 * a.n + i];
+    const int e_hi = a.ck_int[(int64_t)(a.c_hi - a.ck_lo) * 2 * a.n + i];
     const uint8_t *ty = a.syn_type + (int64_t)i * a.n_syn;
     float *gw = a.grad_w + (int64_t)i * a.n_syn;
     for (int s0 = 0; s0 < a.n_syn; s0 += T) {

@@ -4012,8 +4012,11 @@ struct edlut_fit {
     int model = 0, n = 0, steps = 0, n_syn = 0, device = 0;
     FitArgs base{};
     int group = 0;                 // segments the backward pass takes per launch
+    int span = 0;                  // segments it has the states of at once
     float *refr = nullptr;
-    float *ck_state = nullptr;
+    float *kept_state = nullptr;   // the forward pass's checkpoints
+    int32_t *kept_int = nullptr;
+    float *ck_state = nullptr;     // every segment of a span (checkpoints further apart than segments)
     int32_t *ck_int = nullptr;
     double *maps = nullptr, *part = nullptr, *carry = nullptr;
     float *lg = nullptr;
@@ -4022,7 +4025,10 @@ struct edlut_fit {
 
 // Working storage of a backward launch: its segments' maps, partial
 // gradients and conductance adjoints.  Past this the pass takes several
-// launches, last segments first.
+// launches, last segments first.  Checkpoints are kept for every segment up to
+// as much memory, past it as far apart as the caller allows: the backward pass
+// then runs the forward recurrence again between them.  (The V trace and dL/dV
+// take ten times what a checkpoint every 32 steps does.)
 static constexpr size_t kFitScratch = (size_t)256 << 20;
 
 extern "C" {
@@ -4091,14 +4097,19 @@ int edlut_fit_create(int model, const float *params, int n_params, float dt_s, i
     }
     a.refr_len = (int)refr.size();
     const size_t n = (size_t)n_neurons, segs = (size_t)a.segs;
+    const size_t ck_bytes = n * (4 * sizeof(float) + 2 * sizeof(int32_t));
+    a.keep = segs * ck_bytes <= kFitScratch ? 1 : std::max(1, std::min(checkpoint, steps) / a.seg);
+    const size_t keep = (size_t)a.keep, kept = (segs + keep - 1) / keep;
     const size_t per_seg = n * (sizeof(double) * (kFitMap + 4) + sizeof(float) * 2 * a.seg);
     f->group = (int)std::max<size_t>(1, std::min(segs, kFitScratch / per_seg));
-    const size_t group = (size_t)f->group;
+    const size_t group = (size_t)f->group, span = keep > 1 ? std::min(segs, std::max<size_t>(1, group / keep) * keep) : segs;
+    f->span = (int)span;
     int rc;
-    if ((rc = dalloc(&f->refr, refr.size() + 1)) || (rc = dalloc(&f->ck_state, segs * 4 * n)) ||
-        (rc = dalloc(&f->ck_int, (segs + 1) * 2 * n)) || (rc = dalloc(&f->maps, group * kFitMap * n)) ||
+    if ((rc = dalloc(&f->refr, refr.size() + 1)) || (rc = dalloc(&f->kept_state, (kept + 1) * 4 * n)) ||
+        (rc = dalloc(&f->kept_int, (kept + 1) * 2 * n)) || (rc = dalloc(&f->maps, group * kFitMap * n)) ||
         (rc = dalloc(&f->part, group * 4 * n)) || (rc = dalloc(&f->lg, group * a.seg * 2 * n)) ||
-        (rc = dalloc(&f->carry, 8 * n))) {
+        (rc = dalloc(&f->carry, 8 * n)) ||
+        (keep > 1 && ((rc = dalloc(&f->ck_state, span * 4 * n)) || (rc = dalloc(&f->ck_int, (span + 1) * 2 * n))))) {
         edlut_fit_destroy(f);
         return rc;
     }
@@ -4108,8 +4119,10 @@ int edlut_fit_create(int model, const float *params, int n_params, float dt_s, i
         return fail(EDLUT_E_HIP, "hipMemcpy failed");
     }
     a.refr = f->refr;
-    a.ck_state = f->ck_state;
-    a.ck_int = f->ck_int;
+    a.kept_state = f->kept_state;
+    a.kept_int = f->kept_int;
+    a.ck_state = keep > 1 ? f->ck_state : f->kept_state;
+    a.ck_int = keep > 1 ? f->ck_int : f->kept_int;
     a.maps = f->maps;
     a.part = f->part;
     a.lg = f->lg;
@@ -4122,7 +4135,7 @@ int edlut_fit_destroy(edlut_fit *f) {
     if (!f) return 0;
     (void)hipSetDevice(f->device);
     (void)hipDeviceSynchronize();
-    void *dev[] = {f->refr, f->ck_state, f->ck_int, f->maps, f->part, f->lg, f->carry};
+    void *dev[] = {f->refr, f->kept_state, f->kept_int, f->ck_state, f->ck_int, f->maps, f->part, f->lg, f->carry};
     for (void *q : dev)
         if (q) (void)hipFree(q);
     delete f;
@@ -4163,7 +4176,7 @@ int edlut_fit_forward(edlut_fit *f, const edlut_fit_tensors *t, void *stream) {
     if (!t->v_trace) return fail(EDLUT_E_ARG, "v_trace is null");
     HIP_TRY(hipSetDevice(f->device));
     const int blocks = (f->n + kFitBlock - 1) / kFitBlock;
-    const bool extra = t->spikes || t->traj || a.refr_len > kFitRefr;
+    const bool extra = t->spikes || t->traj || a.refr_len > kFitRefr || a.keep > 1;
     auto fn = f->model == EDLUT_LIF ? (extra ? k_fit_forward<0, true> : k_fit_forward<0, false>)
                                     : (extra ? k_fit_forward<1, true> : k_fit_forward<1, false>);
     hipLaunchKernelGGL(fn, dim3(blocks), dim3(2 * kFitBlock), 0, (hipStream_t)stream, a);
@@ -4185,13 +4198,24 @@ int edlut_fit_backward(edlut_fit *f, const edlut_fit_tensors *t, void *stream) {
     // the adjoint state after the last step is zero
     hipLaunchKernelGGL(k_fill_i32, dim3(std::min(neurons, 1024u)), dim3(kBlock), 0, st, (int32_t *)f->carry,
                        (int64_t)(2 * 4) * f->n, 0);
-    for (a.c_hi = a.segs; a.c_hi > 0; a.c_hi = a.c_lo) {
-        a.c_lo = std::max(a.c_hi - f->group, 0);
-        const unsigned blocks = (unsigned)(((int64_t)(a.c_hi - a.c_lo) * f->n + kFitBlock - 1) / kFitBlock);
-        hipLaunchKernelGGL(lif ? k_fit_maps<0> : k_fit_maps<1>, dim3(blocks), dim3(kFitBlock), 0, st, a);
-        hipLaunchKernelGGL(k_fit_scan, dim3(neurons), dim3(kFitBlock), 0, st, a);
-        hipLaunchKernelGGL(lif ? k_fit_sweep<0> : k_fit_sweep<1>, dim3(blocks), dim3(kFitBlock), 0, st, a);
-        hipLaunchKernelGGL(k_fit_grads, dim3((unsigned)f->n), dim3(kFitGradBlock), 0, st, a);
+    for (int hi = a.segs, lo; hi > 0; hi = lo) {
+        // a span of segments, from a kept checkpoint on
+        lo = (std::max(hi - f->span, 0) + a.keep - 1) / a.keep * a.keep;
+        if (a.keep > 1) {
+            a.ck_lo = a.c_lo = lo;
+            a.c_hi = hi;
+            const int64_t kept = (hi - lo + a.keep - 1) / a.keep;
+            const unsigned kb = (unsigned)((kept * f->n + kFitBlock - 1) / kFitBlock);
+            hipLaunchKernelGGL(lif ? k_fit_expand<0> : k_fit_expand<1>, dim3(kb), dim3(kFitBlock), 0, st, a);
+        }
+        for (a.c_hi = hi; a.c_hi > lo; a.c_hi = a.c_lo) {
+            a.c_lo = std::max(a.c_hi - f->group, lo);
+            const unsigned blocks = (unsigned)(((int64_t)(a.c_hi - a.c_lo) * f->n + kFitBlock - 1) / kFitBlock);
+            hipLaunchKernelGGL(lif ? k_fit_maps<0> : k_fit_maps<1>, dim3(blocks), dim3(kFitBlock), 0, st, a);
+            hipLaunchKernelGGL(k_fit_scan, dim3(neurons), dim3(kFitBlock), 0, st, a);
+            hipLaunchKernelGGL(lif ? k_fit_sweep<0> : k_fit_sweep<1>, dim3(blocks), dim3(kFitBlock), 0, st, a);
+            hipLaunchKernelGGL(k_fit_grads, dim3((unsigned)f->n), dim3(kFitGradBlock), 0, st, a);
+        }
     }
     HIP_TRY(hipGetLastError());
     return 0;
