@@ -73,6 +73,7 @@ EXPORTS = (
     "edlut_network_get_stdp",
     "edlut_network_set_launch",
     "edlut_network_get_launch",
+    "edlut_network_pulled_groups",
     "edlut_network_autotune",
     "edlut_fit_create",
     "edlut_fit_destroy",
@@ -170,6 +171,7 @@ def _sig(lib):
         "edlut_network_get_stdp": (I32, [P, I32, P, P, P]),
         "edlut_network_set_launch": (I32, [P, I32, I32, I32]),
         "edlut_network_get_launch": (I32, [P, P, P, P]),
+        "edlut_network_pulled_groups": (I32, [P, P]),
         "edlut_network_autotune": (I32, [P, I32, P, P, P, P]),
         "edlut_fit_create": (I32, [I32, P, I32, F32, I32, I32, I32, I32, I32, P]),
         "edlut_fit_destroy": (I32, [P]),

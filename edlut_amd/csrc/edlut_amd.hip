@@ -3875,6 +3875,19 @@ int edlut_network_get_launch(const edlut_network *n, int *items, int *fold_lanes
 // Times `trial_steps` steps (after 16 warm-up steps) of every launch shape
 // and keeps the fastest; the network is reset before each trial and after
 // the search.  The results of a run do not depend on the launch shape.
+int edlut_network_pulled_groups(edlut_network *n, int *groups) {
+    if (!n || !groups) return fail(EDLUT_E_ARG, "null argument");
+    *groups = -1;
+    if (!n->pull_on) return 0;
+    const PullArgs &a = n->pull;
+    std::vector<uint8_t> m((size_t)a.groups);
+    HIP_TRY(hipSetDevice(n->pop->device));
+    HIP_TRY(hipStreamSynchronize(n->pop->stream));
+    HIP_TRY(hipMemcpy(m.data(), a.mode + (size_t)((n->last_step + 1) & 1) * m.size(), m.size(), hipMemcpyDeviceToHost));
+    *groups = (int)std::count(m.begin(), m.end(), (uint8_t)1);
+    return 0;
+}
+
 int edlut_network_autotune(edlut_network *n, int trial_steps, int *items, int *fold_lanes,
                            int *fold_blocks, double *ms_per_step) {
     if (!n) return fail(EDLUT_E_ARG, "network is null");

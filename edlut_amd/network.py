@@ -225,6 +225,13 @@ class Network:
         C.check(C.lib().edlut_network_get_launch(self._h, C.byref(a), C.byref(b), C.byref(c)))
         return a.value, b.value, c.value
 
+    def pulled_groups(self) -> int:
+        """Groups whose events the next update takes from incoming lists; -1
+        without lists (every event is pushed by its source)."""
+        g = ctypes.c_int(0)
+        C.check(C.lib().edlut_network_pulled_groups(self._h, C.byref(g)))
+        return g.value
+
     def autotune(self, trial_steps: int = 64):
         """Pick the fastest launch shape by timing trial runs (the network is
         reset afterwards).  Returns (items, lanes, blocks, ms_per_step)."""

@@ -418,6 +418,11 @@ int edlut_network_reset(edlut_network *net);
 int edlut_network_set_launch(edlut_network *net, int items, int fold_lanes, int fold_blocks);
 int edlut_network_get_launch(const edlut_network *net, int *items, int *fold_lanes,
                              int *fold_blocks);
+/* Groups of a grouped population whose events the next update takes from
+ * incoming lists (dense firing) instead of pushed by their sources; -1: none
+ * can, no lists were built (before the first run, plastic synapses, synapses
+ * between groups, several sources, long lists).  The results are the same. */
+int edlut_network_pulled_groups(edlut_network *net, int *groups);
 /* Autotuner: times trial_steps steps of every launch shape on this network
  * and keeps the fastest (returned, with its time per step); resets the
  * network before each trial and after the search. */

@@ -71,14 +71,15 @@ def test_mixed_groups(graph, items):
             pnet.close()
             pm.close()
         assert max(rates) > 0.02 and min(rates) < 0.002, rates
+        assert 0 < gnet.pulled_groups() < len(sizes)
         gnet.reset()
 
 
-def _random_edges(rng, n, e, max_d):
-    # duplicates of one (source, target, delay), targets without synapses, hubs
+def _random_edges(rng, n, e, max_d, hub):
+    # duplicates of one (source, target, delay), targets without synapses, a hub
     src = rng.integers(0, n, e).astype(np.int32)
-    tgt = rng.integers(0, max(1, n * 3 // 4), e).astype(np.int32)
-    tgt[: e // 10] = 0
+    tgt = rng.integers(0, max(1, n * 7 // 8), e).astype(np.int32)
+    tgt[: min(hub, e)] = 0
     src[e // 2: e // 2 + e // 8] = src[: e // 8]
     tgt[e // 2: e // 2 + e // 8] = tgt[: e // 8]
     delay = rng.integers(1, max_d + 1, e).astype(np.int32)
@@ -86,17 +87,18 @@ def _random_edges(rng, n, e, max_d):
     return src, tgt, delay, (rng.random(e) < 0.3).astype(np.uint8), rng.lognormal(1.0, 1.0, e).astype(np.float32)
 
 
-@pytest.mark.parametrize("between", [False, True])
-def test_given_synapses(between):
-    """Synapse lists of every length; `between`: some synapses between groups,
-    which keeps delivery with the push fold."""
-    sizes, max_d = [300, 700, 1], 5
-    print(f"case given synapses between={between}", flush=True)
+@pytest.mark.parametrize("lists,hub,between", [(True, 100, False), (False, 100, True), (False, 3000, False)])
+def test_given_synapses(lists, hub, between):
+    """Incoming lists of every length, none and one synapse among them; some
+    synapses between groups, or a hub with more synapses than a list can take,
+    keep delivery with the push fold."""
+    sizes, max_d = [300, 1500, 1], 5
+    print(f"case given synapses lists={lists} hub={hub} between={between}", flush=True)
     params = np.tile(ADEX_DEFAULTS, (3, 1))
     gm, gnet = _group(sizes, params, max_d)
     start, _ = gm.GetGroups()
     rng = np.random.default_rng(4)
-    edges = [_random_edges(rng, n, 40 * n, max_d) for n in sizes]
+    edges = [_random_edges(rng, n, 40 * n, max_d, hub) for n in sizes]
     src = np.concatenate([e[0] + s for e, s in zip(edges, start)])
     tgt = np.concatenate([e[1] + s for e, s in zip(edges, start)])
     rest = [np.concatenate([e[j] for e in edges]) for j in (2, 3, 4)]
@@ -111,9 +113,12 @@ def test_given_synapses(between):
         v[s:s + n] = rng.uniform(-60, -20, n)
     gm.SetVectorNeuronState(0, v)
     pm.SetVectorNeuronState(0, v)
+    pulled = []
     for r in (3, 40, 80):
         gnet.run(r)
         pnet.run(r)
+        pulled.append(gnet.pulled_groups())
+    assert max(pulled) > 0 if lists else set(pulled) == {-1}, pulled
     a, b = gnet.spikes(), pnet.spikes()
     assert len(a[0]) > 0.01 * 123 * gm.size
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
@@ -142,10 +147,12 @@ def test_source_added_between_runs():
     nets = [gnet] + [p[1] for p in alone]
     for net in nets:
         net.run(150)
+        assert net is not gnet or net.pulled_groups() == len(sizes)
         empty = np.zeros(0, np.int32)
         net.add_poisson(np.arange(1, 4, dtype=np.uint32), 0.0,
                         *build_out_csr(3, net.model.size, max_d, empty, empty, empty, empty.astype(np.uint8),
                                        empty.astype(np.float32)))
         net.run(100)
+        assert net.pulled_groups() == -1
     for g, n in enumerate(sizes):
         assert _equal(gm, gnet, g, *alone[g], n) > 0.02
