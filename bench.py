@@ -243,21 +243,22 @@ def bench_sweep(n_networks: int, steps: int, seq_sample: int, seq_steps: int, cp
 
 def bench_adjoint(n: int, steps: int, checkpoint: int, cpu: bool, reps: int = 3):
     """Trace-fitting forward and adjoint kernels (256 LIF/Euler + 256 AdEx/RK4
-    neurons, 50 Poisson inputs at 20 Hz, 10,000 steps, checkpoints every 100
-    steps): kernel time of the backward pass over the forward pass.
+    neurons, 50 Poisson inputs at 20 Hz, 10,000 steps, a checkpoint spacing of
+    100 steps): kernel time of the backward pass over the forward pass.
 
-    Both kernels run one lane per neuron through a sequential recurrence, so
-    they are bound by the latency of each lane's dependent instruction chain:
-    `roofline` compares the measured forward time with the issue time of its
-    VALU instructions on one SIMD (4 cycles per wave64 instruction), from the
-    instruction count of the committed counter profile."""
+    The forward kernel runs one lane per neuron through a sequential
+    recurrence, so it is bound by the latency of each lane's dependent
+    instruction chain: `roofline` compares the measured forward time with the
+    issue time of the recurrence wave's VALU instructions on one SIMD (4 cycles
+    per wave64 instruction), from the instruction count of the committed
+    counter profile."""
     import torch
 
     from edlut_amd import workloads
     from edlut_amd.adjoint import FitProblem
 
     out = {"workload": f"{n} LIF (Euler) + {n} AdEx (RK4) neurons, 50 inputs at 20 Hz, {steps} steps, "
-                       f"checkpoint every {checkpoint}"}
+                       f"checkpoint spacing {checkpoint} (states are kept every 32 steps below 256 MB)"}
     total_f = total_b = 0.0
     specs = {}
     for model, key in (("LIFTimeDrivenModel_GPU", "lif"), ("AdExTimeDrivenModel_GPU", "adex")):
@@ -287,7 +288,7 @@ def bench_adjoint(n: int, steps: int, checkpoint: int, cpu: bool, reps: int = 3)
             issue_ms = instr * 4 / CLOCK_HZ * 1e3
             out[key]["roofline"] = {"bound": "latency", "achieved": issue_ms, "peak": f, "unit": "ms",
                                     "frac": issue_ms / f,
-                                    "basis": "VALU issue time of one wave's forward instructions / forward time"}
+                                    "basis": "VALU issue time of the recurrence wave's forward instructions / forward time"}
         total_f += f
         total_b += b
         prob.close()

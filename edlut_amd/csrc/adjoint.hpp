@@ -43,8 +43,9 @@ namespace edl {
 
 constexpr int kFitBlock = 64;   // neurons (forward) or (segment, neuron) pairs per workgroup
 // Longest segment: the forward pass stages a segment's inputs (four values
-// per step and lane, twice) and the backward pass its states (four values)
-// in LDS: 64 KB and 32 KB, so four backward waves share a CU.
+// per step and lane, twice, one step of padding each: 66 KB, 68 KB with its
+// small tables) and the backward pass its states (four values, 32 KB) in LDS, so
+// two forward workgroups or five backward waves share a CU's 160 KB.
 constexpr int kFitSeg = 32;
 constexpr int kFitRefr = 256;   // refractory fractions staged in LDS (longer tables: read from memory)
 constexpr int kFitGradBlock = 128;

@@ -1302,7 +1302,6 @@ UpdateFn pick_update(const edlut_population *p, bool ext) {
 
 // The error word's message and code.
 int err_code(uint32_t e) {
-    if (e & 1u) return fail(EDLUT_E_STATE, "spike compaction look-back exceeded its spin limit");
     if (e & 2u)
         return fail(EDLUT_E_CAP, "spike log capacity exceeded (read and clear the log between runs, or raise "
                                  "its capacity)");

@@ -525,12 +525,12 @@ __device__ __forceinline__ void eq_window(EqItem *__restrict__ h, const EqArgs &
     flush();
 }
 
-// The replay of one window by one workgroup of kBlock threads: the spikes
-// per delay are counted by all lanes, the heap operations run on the first wave.
 // Spikes that a wave counts together (others, one by one in the lane that
 // loaded their tile's count).
 constexpr int kEqList = 256;
 
+// The replay of one window by one workgroup of kBlock threads: the spikes
+// per delay are counted by all lanes, the heap operations run on the first wave.
 // LDS_ITEMS heap entries are staged in LDS when the heap cannot outgrow
 // them; MAXD bounds the delays (host-checked).
 template <int LDS_ITEMS, int MAXD>

@@ -2,8 +2,8 @@
 // target's side, for the groups that fire densely.
 //
 // The fold (fold_ring_body) pushes every event into its target's segment with
-// scattered atomics and stores, and the update kernel sorts the segment.  Where many sources fire it is cheaper to read every
-// synapse: each target walks its incoming list, which is kept in delivery
+// scattered atomics and stores, and the update kernel sorts the segment.  Where
+// many sources fire it is cheaper to read every synapse: each target walks its incoming list, which is kept in delivery
 // order (delay, source, position in the source's row), and tests the source's
 // bit in a bitmap of the spikes of each delay's update, staged in LDS.  The
 // events that are due are added to the conductance as they come: no atomics,
@@ -53,9 +53,17 @@ struct PullArgs {
 };
 
 // A pulled group reads 8 bytes of every synapse (1.6 ps at the rate of a large
-// copy), a pushed event costs about 0.16 ns with the sorting.  Measured on 512
-// networks, the three kernels per step: 286 us with the line at one neuron in
-// 300 firing per update, 299 us at one in 100, 357 us at one in 30.
+// copy), a pushed event costs about 0.16 ns with the sorting: by those they meet
+// at one neuron in 100 firing per update.  Sweeps, us per step, by the line:
+//
+//   networks, in-degree    1/30   1/100   1/300   1/1,000   1/3,000
+//   512, 25                 124     128     126       115       108
+//   512, 100                344     308     307       306       306
+//   256, 250                610     609     609       608       610
+//
+// From one in 100 down the line hardly matters at in-degree 100 and above (few
+// groups lie between), so 300 stands anywhere on that flat; sparse wiring gains
+// up to 15% from a lower one, as a quiet group's walk is short.
 __device__ __forceinline__ bool pull_dense(uint32_t spikes, int32_t n, int delays) {
     return (uint64_t)spikes * 300ull >= (uint64_t)n * (uint64_t)delays;
 }

@@ -3,7 +3,7 @@ the FP64 adjoint (itself pinned by finite differences), the
 torch.autograd.Function, and the backward/forward cost ratio.
 
 Workload of the contract (config 5): 256 LIF (Euler) and 256 AdEx (RK4)
-neurons, 50 inputs each at 20 Hz, 10,000 steps, checkpoints every 100 steps.
+neurons, 50 inputs each at 20 Hz, 10,000 steps, a checkpoint spacing of 100.
 """
 import numpy as np
 import pytest
