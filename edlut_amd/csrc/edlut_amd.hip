@@ -380,7 +380,6 @@ struct edlut_population {
         t.head = head;
         t.node = node;
         t.n_node = (uint32_t)q_n;
-        t.err = err;
         return t;
     }
 

@@ -14,8 +14,8 @@ struct alignas(8) FoldNode {
 
 // Lists of up to this many events are summed by selection, longer ones sorted
 // first.  An update of one AdEx cell, of 8 and of 64 cells with 96 events on
-// each takes 237, 736 and 508 us by selection, with 97 (sorted) 174, 727 and
-// 513 us.
+// each takes 270, 322 and 482 us by selection, with 97 (sorted) 184, 348 and
+// 532 us.
 constexpr uint32_t kListShort = 96;
 
 // Sorts the list from `hd` by event number: its runs (a wave's events arrive
