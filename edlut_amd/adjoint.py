@@ -45,8 +45,8 @@ class FitProblem:
     syn_type: [n, n_syn] 0 exc / 1 inh; events: (ev_ptr [n+1], ev_step, ev_syn)
     with each neuron's events sorted by step (ev_step = the update they precede).
     checkpoint: steps between the states the forward pass keeps for the backward
-    pass; a spacing above 32 saves memory once a state every 32 steps would take
-    more than 256 MB, and is not used before.
+    pass.  A spacing above 32 (rounded down to a multiple of 32) saves memory once
+    a state every 32 steps would take more than 256 MB, and is not used before.
     """
 
     def __init__(self, model: str, params, n: int, steps: int, syn_type, events, dt_s=1e-4,

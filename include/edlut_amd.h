@@ -437,8 +437,9 @@ int edlut_network_autotune(edlut_network *net, int trial_steps, int *items, int 
  * dt_s.  params holds the model's parameter vector (order of
  * edlut_population_create); g_leak, e_leak, tau_exc and tau_inh are taken
  * per neuron from the tensors instead.  The forward pass writes the V trace
- * and keeps the state every `checkpoint` steps, or (where that is less memory
- * than 256 MB) every 32 steps if `checkpoint` is more; the backward pass takes
+ * and keeps the state every `checkpoint` steps (above 32, rounded down to a
+ * multiple of 32), or every 32 steps if `checkpoint` is more and that takes at
+ * most 256 MB; the backward pass takes
  * dL/dV for every step and writes dL/d(g_leak, e_leak, tau_exc, tau_inh)
  * per neuron and dL/dweight per synapse.  It is the reverse-mode derivative
  * of the discrete forward map, with the forward run's spike pattern held
